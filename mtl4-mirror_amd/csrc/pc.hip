@@ -14,6 +14,7 @@
 #include "m4g_device.hpp"
 #include "pc.hpp"
 #include "krylov.hpp"
+#include "sentinel.hpp"
 
 #include <algorithm>
 #include <future>
@@ -24,24 +25,6 @@
 #include <cstdlib>
 
 namespace m4g {
-
-// ---------------------------------------------------------------------------
-// sentinels of the sweep exchange buffers: signalling NaNs, which arithmetic
-// never produces (results that are NaN come out quiet)
-// ---------------------------------------------------------------------------
-template <typename T> struct Sentinel;
-template <> struct Sentinel<double> {
-    static constexpr uint64_t bits = 0x7FF0DEADBEEF0001ull;
-    __device__ static double value() { return __longlong_as_double((long long)bits); }
-    __device__ static bool is(double v) { return (uint64_t)__double_as_longlong(v) == bits; }
-    __device__ static double canon(double v) { return is(v) ? __longlong_as_double(0x7FF8000000000000ll) : v; }
-};
-template <> struct Sentinel<float> {
-    static constexpr uint32_t bits = 0x7F80BEEFu;
-    __device__ static float value() { return __int_as_float((int)bits); }
-    __device__ static bool is(float v) { return (uint32_t)__float_as_int(v) == bits; }
-    __device__ static float canon(float v) { return is(v) ? __int_as_float(0x7FC00000) : v; }
-};
 
 // ---------------------------------------------------------------------------
 // factorisation kernels
@@ -826,8 +809,33 @@ static void build_recs_w(SweepDev& d, int vbytes, hipStream_t s)
     }
 }
 
+void SweepDev::init_line(const LineGeom& G, int kind, int ftype, const double* f, const int32_t* frows)
+{
+    line = std::make_unique<LineSweep>();
+    line->init(G, kind, ftype, f, frows);
+    factor_type = ftype;
+    SweepPlan p;
+    p.n = G.n();
+    p.lower = !line_upper(kind);
+    p.unit = line_unit(kind);
+    p.width = 2;
+    p.ntiles = G.strips;
+    p.max_steps = G.steps;
+    p.levels = int64_t(G.nx) + G.ny - 1;
+    p.shape.grid = true;
+    p.shape.e1 = 1;
+    p.shape.e2 = 64;
+    p.shape.e3 = G.nx;
+    plan_meta = p;
+}
+
 void SweepDev::refresh_values(const double* f, int ftype)
 {
+    if (line) {
+        line->fstore = f;
+        line->stale = true;
+        return;
+    }
     // records are packed at the next launch, for that launch's vector type
     factor_type = ftype;
     fsrc = f;
@@ -947,6 +955,21 @@ void run_sweep_pair(SweepDev& first, SweepDev& second, const void* v, void* tmp,
                     const int* skip, hipStream_t s, const void* dot_with, double* dot_partials)
 {
     M4G_REQUIRE(first.factor_type == second.factor_type, M4G_ERR_INVALID, "sweep factor types differ");
+    if (first.line) {
+        M4G_REQUIRE(second.line, M4G_ERR_LOGIC, "sweep forms differ");
+        M4G_REQUIRE(first.factor_type == M4G_F32 || vtype == M4G_F64, M4G_ERR_INVALID,
+                    "double factors need double vectors");
+        first.line->prepare(vtype, s);
+        second.line->prepare(vtype, s);
+        for (int dir = 0; dir < 2; dir++) {
+            SweepDev& d = dir ? second : first;
+            const SweepPlan& p = d.plan_meta;
+            TraceRange tr(!p.lower ? kTraceUpperTrisolve : p.unit ? kTraceLowerUnitTrisolve : kTraceLowerTrisolve);
+            d.line->launch(dir ? *first.line : *second.line, dir ? tmp : v, dir ? y : tmp, vtype, skip, spin_limit(),
+                           dir ? dot_with : nullptr, dir ? dot_partials : nullptr, s);
+        }
+        return;
+    }
     first.ensure_exchange(vtype);
     second.ensure_exchange(vtype);
     if (first.factor_type == M4G_F64) {
@@ -1016,10 +1039,11 @@ bool pc_grid_factor(m4g_pc_s& P, int64_t max_n, DevBuf<double>& east, DevBuf<dou
 int check_sweep_fault(SweepDev& d)
 {
     int h = 0;
-    M4G_HIP(hipMemcpyAsync(&h, d.fault.ptr, sizeof(int), hipMemcpyDeviceToHost, current_stream()));
+    int* fault = d.line ? d.line->fault.ptr : d.fault.ptr;
+    M4G_HIP(hipMemcpyAsync(&h, fault, sizeof(int), hipMemcpyDeviceToHost, current_stream()));
     M4G_HIP(hipStreamSynchronize(current_stream()));
     if (h) {
-        M4G_HIP(hipMemsetAsync(d.fault.ptr, 0, sizeof(int), current_stream()));
+        M4G_HIP(hipMemsetAsync(fault, 0, sizeof(int), current_stream()));
         M4G_HIP(hipStreamSynchronize(current_stream()));
     }
     return h;
@@ -1331,12 +1355,30 @@ int m4g_pc_create(m4g_pc* out, m4g_matrix A, int kind, int ftype)
             P->grid = g;
             // the sweep plans need only the pattern: they are built on host
             // threads while this thread runs the factorisation on the device
-            const int64_t cap = sweep_tile_cap(ftype == M4G_F64 ? M4G_F64 : M4G_F32);
-            PlanPairJob plans(lo, up, g, cap, ftype, &lo_levels);
-            factorize_levels(*P, lo, *A, lo_levels);
-            mark("factor");
-            plans.finish(P->lower, P->upper, P->fstore.ptr);
-            mark("plan+upload");
+            // a 2D grid with the whole 5-point pattern: line sweeps, which need no plan (256 x 256: 30 us a sweep
+            // against 88; 64 x 64: 9 against 27).  They need a line's steps in LDS (line_geometry).
+            P->line = LineGeom();
+            if (g.nz == 1 && star_pattern(g, n, P->fS.data(), P->fI.data(), kind == M4G_PC_IC0))
+                P->line = line_geometry(g, sweep_lds_budget());
+            if (P->line.strips) {
+                factorize_levels(*P, lo, *A, lo_levels);
+                mark("factor");
+                std::vector<int32_t> rows(P->fS.begin(), P->fS.end());
+                P->frows.reset(rows.size());
+                P->frows.upload(rows.data(), rows.size());
+                const bool ic = kind == M4G_PC_IC0;
+                P->lower.init_line(P->line, ic ? kLineIc0Lower : kLineIluLower, ftype, P->fstore.ptr, P->frows.ptr);
+                P->upper.init_line(P->line, ic ? kLineIc0Upper : kLineIluUpper, ftype, P->fstore.ptr, P->frows.ptr);
+                M4G_HIP(hipStreamSynchronize(s));   // `rows` is read by the copy
+                mark("lines");
+            } else {
+                const int64_t cap = sweep_tile_cap(ftype == M4G_F64 ? M4G_F64 : M4G_F32);
+                PlanPairJob plans(lo, up, g, cap, ftype, &lo_levels);
+                factorize_levels(*P, lo, *A, lo_levels);
+                mark("factor");
+                plans.finish(P->lower, P->upper, P->fstore.ptr);
+                mark("plan+upload");
+            }
             P->tmp_bytes = 0;
         }
         M4G_HIP(hipStreamSynchronize(s));
@@ -1437,6 +1479,11 @@ void pc_apply(m4g_pc_s& P, const void* x, void* y, int vtype, bool adjoint, hipS
     if (n == 0) return;
     void* tmp = pc_tmp(P, vtype);
     if (adjoint && P.kind == M4G_PC_ILU0) {
+        if (!P.adj_ready && P.line.strips) {
+            P.adj_lower.init_line(P.line, kLineAdjLower, P.factor_type, P.fstore.ptr, P.frows.ptr);
+            P.adj_upper.init_line(P.line, kLineAdjUpper, P.factor_type, P.fstore.ptr, P.frows.ptr);
+            P.adj_ready = true;
+        }
         if (!P.adj_ready) {
             SweepRows lo, up;
             M4G_REQUIRE(ilu0_adjoint_rows(n, P.fS.data(), P.fI.data(), lo, up), M4G_ERR_MISSING_DIAGONAL,

@@ -1,6 +1,7 @@
 // Preconditioner handle and compiled sweeps (device side).
 #pragma once
 
+#include "lines.hpp"
 #include "m4g_internal.hpp"
 #include "schedule.hpp"
 
@@ -25,7 +26,10 @@ struct SweepDev {
     DevBuf<unsigned> tickets;
     DevBuf<int> fault;
     int factor_type = M4G_F64;
+    // a 5-point grid factor: the line sweep that takes the place of all of the above but plan_meta's scalars
+    std::unique_ptr<LineSweep> line;
 
+    void init_line(const LineGeom& G, int kind, int ftype, const double* fstore_dev, const int32_t* frows_dev);
     void upload(const SweepPlan& p, const double* fstore_dev, int ftype);
     void refresh_values(const double* fstore_dev, int ftype);
     void ensure_recs(int vbytes, hipStream_t s);
@@ -61,6 +65,8 @@ struct m4g_pc_s {
     m4g::DevBuf<double> fstore;
     m4g::DevBuf<int32_t> a_pos;           // IC(0): CSR index in A of each upper(A) entry
     m4g::DevBuf<double> inv_diag;         // diagonal PC
+    m4g::LineGeom line;                   // strips of the line sweeps (strips 0: the general sweeps)
+    m4g::DevBuf<int32_t> frows;           // line sweeps: row starts of the factor storage
     m4g::SweepDev lower, upper;           // solve: lower then upper
     m4g::SweepDev adj_lower, adj_upper;   // ILU(0) adjoint_solve
     bool adj_ready = false;

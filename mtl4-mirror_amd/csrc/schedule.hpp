@@ -60,6 +60,11 @@ struct GridInfo {
 };
 GridInfo infer_grid(int64_t n, const int64_t* starts, const int64_t* indices);
 
+// True when every row of the pattern holds exactly its in-grid neighbours of
+// the 5-point (nz == 1) or 7-point stencil and its diagonal, in column order;
+// upper_only: the diagonal and the neighbours after it.
+bool star_pattern(const GridInfo& g, int64_t n, const int64_t* starts, const int64_t* indices, bool upper_only);
+
 // One row of a sweep: entries in the order they are subtracted, with the
 // factor-storage index of each value and of the diagonal (-1: unit diagonal).
 // Rows and factor-storage indices are 32-bit: the builders below reject a

@@ -1,0 +1,111 @@
+"""Triangular sweeps of 5-point grid factors at the sizes where their strips can
+go wrong: fewer lines than a wavefront's, exact multiples and one past them,
+lines shorter than the lanes' skew, long lines (7-point grids beside them).
+IC(0) and ILU(0), both directions and the adjoint, equal the oracle's bit for
+bit (each row's operations run in the reference's order), also with single
+precision factors, with infinities and NaN in the right-hand side, after a
+refactorisation, and in the r.z partials of the last sweep."""
+import numpy as np
+import pytest
+
+import oracle_lib as o
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def g():
+    import mtl4gpu
+    return mtl4gpu
+
+
+def star(nx, ny, nz, seed):
+    """A 5-point (nz == 1) or 7-point matrix with random nonsymmetric entries, diagonally dominant."""
+    rng = np.random.default_rng(seed)
+    r = np.arange(nx * ny * nz)
+    i, j, k = r % nx, r // nx % ny, r // (nx * ny)
+    offs = [(-nx * ny, k > 0), (-nx, j > 0), (-1, i > 0), (0, r >= 0), (1, i < nx - 1), (nx, j < ny - 1),
+            (nx * ny, k < nz - 1)]
+    keep = np.stack([m for _, m in offs], axis=1)
+    cols = np.stack([r + d for d, _ in offs], axis=1)
+    vals = -rng.uniform(0.1, 1.0, keep.shape)
+    vals[:, 3] = 6.5 + rng.uniform(0.0, 1.0, len(r))
+    S = np.concatenate([[0], np.cumsum(keep.sum(axis=1))]).astype(np.int64)
+    return S, cols[keep], vals[keep]
+
+
+SHAPES = [(2, 2, 1), (7, 3, 1), (64, 64, 1), (5, 65, 1), (130, 64, 1), (33, 128, 1), (40, 129, 1), (301, 173, 1),
+          (700, 70, 1), (9, 700, 1), (3600, 66, 1), (4, 4, 4), (20, 33, 9)]
+
+
+def apply(g, P, v, dtype=np.float64, adjoint=False):
+    x, y = g.Vector(data=v, dtype=dtype), g.Vector(len(v), dtype=dtype)
+    (P.adjoint_solve if adjoint else P.solve)(x, y)
+    return y.numpy()
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_line_sweeps_equal_the_oracle(g, shape):
+    print(f"line sweeps {shape}", flush=True)
+    S, I, V = star(*shape, seed=sum(shape))
+    A = o.CSR(S, I, V)
+    v = g.rng_uniform(3, 1, A.n)
+    Ag = g.Matrix(S, I, V)
+    st, L, U = o.ilu0_factor(A)
+    P = g.PC(Ag, g.PC_ILU0)
+    for _ in range(2):   # the exchange buffers are reset by the sweeps themselves
+        np.testing.assert_array_equal(apply(g, P, v), o.ilu0_solve(L, U, v))
+        np.testing.assert_array_equal(apply(g, P, v, adjoint=True), o.ilu0_adjoint_solve(L, U, v))
+    st, Uc, Lc = o.ic0_factor(A)
+    P = g.PC(Ag, g.PC_IC0)
+    np.testing.assert_array_equal(apply(g, P, v), o.ic0_solve(Lc, Uc, v))
+    P32 = g.PC(Ag, g.PC_IC0, np.float32)
+    np.testing.assert_array_equal(apply(g, P32, v), o.ic0_solve(Lc, Uc, v, factor_dtype=np.float32))
+    # new values, same pattern
+    S, I, V = star(*shape, seed=sum(shape) + 1)
+    A = o.CSR(S, I, V)
+    Ag.set_values(V)
+    P.refactor(Ag)
+    st, Uc, Lc = o.ic0_factor(A)
+    np.testing.assert_array_equal(apply(g, P, v), o.ic0_solve(Lc, Uc, v))
+
+
+@pytest.mark.parametrize("shape", [(70, 140, 1), (20, 33, 9)])
+def test_line_sweeps_keep_infinities_and_nans_where_they_belong(g, shape):
+    print(f"special values {shape}", flush=True)
+    S, I, V = star(*shape, seed=1)
+    A = o.CSR(S, I, V)
+    st, L, U = o.ilu0_factor(A)
+    P = g.PC(g.Matrix(S, I, V), g.PC_ILU0)
+    for value in (np.inf, -np.inf, np.nan, -0.0):
+        v = g.rng_uniform(3, 1, A.n)
+        v[[A.n // 3, A.n - 2]] = value
+        ref, refa = o.ilu0_solve(L, U, v), o.ilu0_adjoint_solve(L, U, v)
+        np.testing.assert_array_equal(apply(g, P, v), ref)
+        np.testing.assert_array_equal(apply(g, P, v, adjoint=True), refa)
+    z = np.full(A.n, -0.0)
+    np.testing.assert_array_equal(np.signbit(apply(g, P, z)), np.signbit(o.ilu0_solve(L, U, z)))
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 1), (45, 130, 1), (20, 33, 9)])
+def test_line_sweeps_single_precision_vectors(g, shape):
+    # float factors and vectors: the operations of the double sweeps in float
+    print(f"float vectors {shape}", flush=True)
+    S, I, V = star(*shape, seed=2)
+    A = o.CSR(S, I, V)
+    st, U, L = o.ic0_factor(A)
+    v = g.rng_uniform(3, 1, A.n).astype(np.float32)
+    P = g.PC(g.Matrix(S, I, V), g.PC_IC0, np.float32)
+    L32, U32 = [m.data.astype(np.float32) for m in (L, U)]
+    y = v.copy()
+    for r in range(A.n):
+        acc = y[r]
+        for p in range(L.starts[r], L.starts[r + 1] - 1):
+            acc = np.float32(acc - np.float32(L32[p] * y[L.indices[p]]))
+        y[r] = acc * L32[L.starts[r + 1] - 1]
+    for r in range(A.n - 1, -1, -1):
+        acc = y[r]
+        for p in range(U.starts[r] + 1, U.starts[r + 1]):
+            acc = np.float32(acc - np.float32(U32[p] * y[U.indices[p]]))
+        y[r] = acc * U32[U.starts[r]]
+    np.testing.assert_array_equal(apply(g, P, v, dtype=np.float32), y)
