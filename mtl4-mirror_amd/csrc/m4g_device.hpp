@@ -18,6 +18,9 @@ __device__ inline void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// The SIMD (0..3) of its compute unit that a wavefront runs on.
+__device__ inline int simd_id() { return __builtin_amdgcn_s_getreg((1 << 11) | (4 << 6) | 4); }   // HW_ID, bits 5:4
+
 // Butterfly sum over the 64 lanes of a wavefront; every lane gets the total.
 // The combination order is fixed, so results are deterministic.
 __device__ inline double wave_sum(double v)

@@ -209,13 +209,14 @@ struct SweepArgs {
     double* dot_partials;             // [ntiles] per tile: sum of w_r * y_r over its rows
 };
 
-// Workgroup roles: wavefront 0 imports, 1 computes, 2 and 3 load records,
-// 4 exports; all five move rows between HBM and LDS at the start and end.
-constexpr int kSweepWaves = 5;
+// Workgroup roles: one wavefront imports, one computes, two load records, one
+// exports; all eight move rows between HBM and LDS at the start and end.
+constexpr int kSweepWaves = 8;
 constexpr int kSweepThreads = kSweepWaves * kWave;
-constexpr int kImportDepth = 4;       // imports each importer lane polls per window
-constexpr int kFillUnroll = 26;       // row values each thread moves at once between HBM and LDS
-constexpr int kFillLists = 8;         // import and export list entries per thread in the first fill pass
+constexpr int kImportDepth = 2;       // imports each importer lane polls at a time
+constexpr int kImportPolls = 3;       // polls in flight
+constexpr int kFillUnroll = 16;       // row values each thread moves at once between HBM and LDS
+constexpr int kFillLists = 5;         // import and export list entries per thread in the first fill pass
 
 // Byte offsets of the dynamic LDS regions of a sweep workgroup: header (the
 // workgroup's counters), values (rows, imports, one zero), group table, export
@@ -291,20 +292,43 @@ __device__ inline void wait_lds_at_least(int* p, int target)
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// One workgroup per tile (ticket order), five wavefronts with fixed roles,
+// Roles of a tile's wavefronts.  The compute wavefront's pace is its number of
+// instructions (about 7 cycles each, alone on its SIMD), and a wavefront that
+// polls beside it slows it; the hardware spreads the eight wavefronts over the
+// four SIMDs evenly, but in no fixed order.  So each says which SIMD it is on, and
+// the other roles go to wavefronts away from wavefront 0, which computes.
+enum SweepRole { kRoleCompute, kRoleImport, kRoleLoad0, kRoleLoad1, kRoleExport, kRoleIdle };
+__device__ inline int sweep_role(const int* simd, int wave)
+{
+    if (wave == 0) return kRoleCompute;
+    int before = 0;   // wavefronts that choose first: those on other SIMDs, in order
+    for (int x = 1; x < kSweepWaves; x++) {
+        const bool away_x = simd[x] != simd[0], away = simd[wave] != simd[0];
+        before += away_x == away ? x < wave : away_x;
+    }
+    return before < 4 ? kRoleImport + before : int(kRoleIdle);
+}
+
+// One workgroup per tile (ticket order), wavefronts with fixed roles,
 // communicating through LDS counters:
-//  0  importer: polls the tile's imports from earlier tiles (exchange buffer
+//     importer: polls the tile's imports from earlier tiles (exchange buffer
 //     -> LDS) in first-use order; publishes how many have arrived;
-//  1  compute: walks the tile's groups from LDS alone; once a group's
+//     compute: walks the tile's groups from LDS alone; once a group's
 //     records and the imports it needs are present, computes one piece per
 //     lane:  rr = (slot); rr -= L_rj * y_j in stored order; rr *= d_r
 //     (lower_trisolve.hpp:191-209 / 172-189, upper_trisolve.hpp:159-176);
 //     publishes how many groups are finished;
-//  2,3 loaders: stream the tile's piece records into the LDS ring;
-//  4  exporter: stores the finished rows that later tiles read into the
+//     loaders (two): stream the tile's piece records into the LDS ring;
+//     exporter: stores the finished rows that later tiles read into the
 //     exchange buffer.
 // The compute wavefront so issues no global memory operation: its pace is
-// set by LDS and arithmetic latency only.
+// set by LDS and arithmetic latency only.  A sweep is bound by its chain of
+// dependent steps and of hand-overs between tiles, not by bytes.  Eight
+// wavefronts with the roles placed by SIMD and three polls in flight, against
+// five wavefronts in fixed roles with one poll at a time (two IC(0)/ILU(0) sweeps
+// in double, median of one): 7-point grid of 128^3 140.7 -> 128.3 us, 27-point
+// grid of 96^3 315.8 -> 284.4 us (with rows in one piece of 13, see
+// sweep_piece_width), a mesh of 64 400 vertices 174.3 -> 174.9 us.
 template <typename FV, typename VT, bool UNIT, int W>
 __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4* __restrict__ recs,
                                                          const VT* __restrict__ v, VT* __restrict__ y, VT* xbuf,
@@ -335,9 +359,9 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4
     int& finished = hdr[3];       // groups the compute wavefront has finished
     int* half_batch = hdr + 4;    // batch held by each ring half
     const int tid = threadIdx.x, lane = tid % kWave;
-    // the role of a wavefront is uniform: keep its branches scalar, so the
-    // roles' code is not linearised into one another
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    int* simds = hdr + 8;         // the SIMD of each wavefront
+    if (lane == 0) simds[wave] = simd_id();
     // Tiles go out in ticket order, so a tile's dependencies are held by
     // workgroups that have started.  Workgroup 0 is dispatched first and
     // takes tile 0 without a ticket: the first tile, whose start-up is on the
@@ -426,74 +450,85 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4
     }
     __syncthreads();
 
-    if (wave == 0) {
+    // the role of a wavefront is uniform: keep its branches scalar, so the
+    // roles' code is not linearised into one another
+    const SweepRole role = SweepRole(__builtin_amdgcn_readfirstlane(sweep_role(simds, wave)));
+    if (role == kRoleImport) {
         // ---- importer ----
         // Polls the next imports of the tile, in first-use order, straight
         // from the exchange buffer into LDS and publishes the prefix that has
-        // arrived: a window of 64 * kImportDepth after progress, 64 while
-        // waiting (fewer loads on memory that is being written).  A poll
-        // that finds nothing new touches no LDS (the window's slots stay in
-        // registers, the first missing import comes from ballots), so it
-        // does not queue behind the compute wavefront's LDS traffic.
+        // arrived.  Each poll reads the 64 * kImportDepth after progress;
+        // kImportPolls are in flight, because a tile that runs at the pace of
+        // the one before ends up behind by the longest time a value takes,
+        // and that includes the time between two polls.  A poll that finds
+        // nothing new touches no LDS (the window's slots stay in registers,
+        // the first missing import comes from ballots), so it does not queue
+        // behind the compute wavefront's LDS traffic.
         const int32_t* slot_of = reinterpret_cast<const int32_t*>(imp);
         int head = 0;
         int64_t polls = 0;
-        bool wide = true;
-        int32_t xs[kImportDepth];   // exchange slot of import head + lane + 64u; -1: not polled
+        int32_t xs[kImportDepth];   // exchange slot of import head + lane + 64u; -1: none
         auto read_slots = [&]() {
 #pragma unroll
             for (int u = 0; u < kImportDepth; u++) {
                 const int idx = head + lane + kWave * u;
-                xs[u] = idx < ni && (u == 0 || wide) ? slot_of[idx * (sizeof(VT) / 4)] : -1;
+                xs[u] = idx < ni ? slot_of[idx * (sizeof(VT) / 4)] : -1;
             }
         };
-        read_slots();
-        while (head < ni) {
-            VT val[kImportDepth];
+        int from[kImportPolls];
+        VT val[kImportPolls][kImportDepth];
+        auto poll = [&](int k) {   // (every lane loads, those without a slot the first: no branch around a load)
+            from[k] = head;
 #pragma unroll
             for (int u = 0; u < kImportDepth; u++)
-                val[u] = xs[u] >= 0 ? __hip_atomic_load(xbuf + xs[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                    : VT(0);
-            // smallest index of the window that has not arrived (uniform)
-            int first_missing = min(ni, head + kWave * (wide ? kImportDepth : 1));
+                val[k][u] = __hip_atomic_load(xbuf + max(xs[u], 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        read_slots();
+        if (ni)
 #pragma unroll
-            for (int u = kImportDepth - 1; u >= 0; u--) {
-                const unsigned long long miss = __ballot(xs[u] >= 0 && Sentinel<VT>::is(val[u]));
-                if (miss) first_missing = head + kWave * u + int(__builtin_ctzll(miss));
-            }
+            for (int k = 0; k < kImportPolls; k++) poll(k);
+        while (head < ni) {
 #pragma unroll
-            for (int u = 0; u < kImportDepth; u++) {
-                const int idx = head + lane + kWave * u;
-                if (xs[u] >= 0 && idx < first_missing) imp[idx] = val[u];
-            }
-            if (first_missing > head) {
-                head = first_missing;
-                wide = true;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                if (lane == 0) __hip_atomic_store(&progress, head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                read_slots();   // the values written above lie below head
-                continue;
-            }
-            if (wide) {   // nothing new: poll the first 64 only
-                wide = false;
+            for (int k = 0; k < kImportPolls; k++) {
+                // end of the arrived prefix as this poll saw it (uniform)
+                int got = min(ni, from[k] + kWave * kImportDepth);
 #pragma unroll
-                for (int u = 1; u < kImportDepth; u++) xs[u] = -1;
-            }
-            ++polls;
-            if (polls > a.spin_limit ||
-                ((polls & 63) == 0 && __hip_atomic_load(a.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-                // give up: flag the fault and release the compute wavefront
-                // (its results are then meaningless; the host reports the fault)
-                if (lane == 0) {
-                    __hip_atomic_store(a.fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(&progress, ni, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                for (int u = kImportDepth - 1; u >= 0; u--) {
+                    const unsigned long long miss =
+                        __ballot(from[k] + lane + kWave * u < ni && Sentinel<VT>::is(val[k][u]));
+                    if (miss) got = from[k] + kWave * u + int(__builtin_ctzll(miss));
                 }
-                break;
+                if (got > head) {
+#pragma unroll
+                    for (int u = 0; u < kImportDepth; u++) {
+                        // (entries below head hold their values already, and nobody's slots)
+                        const int idx = from[k] + lane + kWave * u;
+                        if (idx >= head && idx < got) imp[idx] = val[k][u];
+                    }
+                    head = got;
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                    if (lane == 0) __hip_atomic_store(&progress, head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    read_slots();   // the values written above lie below head
+                } else if (head < ni) {
+                    ++polls;
+                    if (polls > a.spin_limit ||
+                        ((polls & 63) == 0 && __hip_atomic_load(a.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                        // give up: flag the fault and release the compute wavefront
+                        // (its results are then meaningless; the host reports the fault)
+                        head = ni;
+                        if (lane == 0) {
+                            __hip_atomic_store(a.fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            __hip_atomic_store(&progress, ni, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
+                    }
+                    __builtin_amdgcn_s_sleep(1);
+                }
+                poll(k);
             }
-            __builtin_amdgcn_s_sleep(2);
         }
-    } else if (wave == 1) {
+    } else if (role == kRoleCompute) {
         // ---- compute ----
+        __builtin_amdgcn_s_setprio(3);
         // Batch by batch: wait for the batch's records in the ring, then its
         // groups unrolled.  The next group's record is read from LDS while
         // the current group computes.  Lanes past a group's size hold a copy
@@ -554,7 +589,8 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4
                 __hip_atomic_store(&finished, b * B + j + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
         }
-    } else if (wave == 4) {
+        __builtin_amdgcn_s_setprio(0);
+    } else if (role == kRoleExport) {
         // ---- exporter ----
         // Follows the compute wavefront and stores each finished exported row
         // (in finish order, so exchange slots xb, xb+1, ...) for later tiles.
@@ -573,9 +609,9 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4
                                    __HIP_MEMORY_SCOPE_AGENT);
             e = avail;
         }
-    } else {
-        // ---- loaders: wavefront 2 fills ring half 0, wavefront 3 half 1 ----
-        const int k = wave - 2;
+    } else if (role != kRoleIdle) {
+        // ---- loaders: one fills ring half 0, the other half 1 ----
+        const int k = role - kRoleLoad0;
         const i32x4* rv = reinterpret_cast<const i32x4*>(recs);
         i32x4* rr = reinterpret_cast<i32x4*>(ring);
         i32x4 bufA[B][C], bufB[B][C];
@@ -804,6 +840,7 @@ static void build_recs_w(SweepDev& d, int vbytes, hipStream_t s)
     case 3: build_recs_t<FV, 3>(d, vbytes, s); break;
     case 4: build_recs_t<FV, 4>(d, vbytes, s); break;
     case 8: build_recs_t<FV, 8>(d, vbytes, s); break;
+    case 13: build_recs_t<FV, 13>(d, vbytes, s); break;
     case 16: build_recs_t<FV, 16>(d, vbytes, s); break;
     default: throw Error(M4G_ERR_LOGIC, "unsupported sweep piece width");
     }
@@ -941,6 +978,7 @@ static void launch_sweep_t(SweepDev& d, SweepDev& other, const VT* v, VT* y, con
         case 3: launch_sweep_w<FV, VT, U, 3>(d, a, v, y, xo, skip, s); break;
         case 4: launch_sweep_w<FV, VT, U, 4>(d, a, v, y, xo, skip, s); break;
         case 8: launch_sweep_w<FV, VT, U, 8>(d, a, v, y, xo, skip, s); break;
+        case 13: launch_sweep_w<FV, VT, U, 13>(d, a, v, y, xo, skip, s); break;
         case 16: launch_sweep_w<FV, VT, U, 16>(d, a, v, y, xo, skip, s); break;
         default: throw Error(M4G_ERR_LOGIC, "unsupported sweep piece width");
         }
