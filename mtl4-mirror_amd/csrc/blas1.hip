@@ -111,6 +111,20 @@ __global__ void __launch_bounds__(64) k_post(const double* __restrict__ src, int
     if (threadIdx.x == 0) post_scalars(box, src, count, seq);
 }
 
+// the union of the flags, which it clears, posted to the host
+__global__ void __launch_bounds__(64) k_post_faults(FaultFlags f, HostPost* box, unsigned seq)
+{
+    if (threadIdx.x != 0) return;
+    int any = 0;
+    for (int k = 0; k < f.count; k++) {
+        const int h = *f.flag[k];
+        if (h) *f.flag[k] = 0;
+        any |= h;
+    }
+    const double v = any;
+    post_scalars(box, &v, 1, seq);
+}
+
 void launch_sum_partials(const double* partials, int nblocks, double* out, hipStream_t s)
 {
     hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, s, partials, nblocks, out, nullptr, 0u);
@@ -120,6 +134,12 @@ void launch_post(const double* src, int count, HostPost* box, unsigned seq, hipS
 {
     M4G_REQUIRE(count >= 0 && count <= kPostMax, M4G_ERR_INVALID, "launch_post: too many scalars");
     hipLaunchKernelGGL(k_post, dim3(1), dim3(64), 0, s, src, count, box, seq);
+    M4G_HIP(hipGetLastError());
+}
+
+void launch_post_faults(const FaultFlags& f, HostPost* box, unsigned seq, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_post_faults, dim3(1), dim3(64), 0, s, f, box, seq);
     M4G_HIP(hipGetLastError());
 }
 

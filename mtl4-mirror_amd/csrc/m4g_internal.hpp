@@ -269,5 +269,11 @@ void launch_dot_post(int64_t n, const double* x, const double* y, double* out, H
 void launch_sumsq_post(int64_t n, const double* x, double* out, HostPost* box, unsigned seq, hipStream_t s);
 // posts src[0..count) (count <= kPostMax, device memory) into box with seq
 void launch_post(const double* src, int count, HostPost* box, unsigned seq, hipStream_t s);
+// posts the union of the flags (device memory) into box with seq and clears them
+struct FaultFlags {
+    int* flag[4];
+    int count;
+};
+void launch_post_faults(const FaultFlags& f, HostPost* box, unsigned seq, hipStream_t s);
 
 }  // namespace m4g

@@ -109,3 +109,22 @@ def test_line_sweeps_single_precision_vectors(g, shape):
             acc = np.float32(acc - np.float32(U32[p] * y[U.indices[p]]))
         y[r] = acc * U32[U.starts[r]]
     np.testing.assert_array_equal(apply(g, P, v, dtype=np.float32), y)
+
+
+def test_a_wait_that_gave_up_is_reported_by_each_direction_and_cleared(g, monkeypatch):
+    # one poll per wait: the strips after the first give up, and every wave still ends
+    print("line sweeps with a one-poll limit", flush=True)
+    S, I, V = star(300, 200, 1, seed=4)
+    A = o.CSR(S, I, V)
+    st, L, U = o.ilu0_factor(A)
+    P = g.PC(g.Matrix(S, I, V), g.PC_ILU0)
+    v = g.rng_uniform(3, 1, A.n)
+    for adjoint, ref in ((False, o.ilu0_solve(L, U, v)), (True, o.ilu0_adjoint_solve(L, U, v))):
+        np.testing.assert_array_equal(apply(g, P, v, adjoint=adjoint), ref)
+        with monkeypatch.context() as m:
+            m.setenv("M4G_SPIN_LIMIT", "1")
+            with pytest.raises(g.M4GError) as e:
+                apply(g, P, v, adjoint=adjoint)
+            assert e.value.status == g.ERR_TIMEOUT
+        for _ in range(2):
+            np.testing.assert_array_equal(apply(g, P, v, adjoint=adjoint), ref)
