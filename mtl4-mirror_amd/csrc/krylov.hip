@@ -358,9 +358,10 @@ __global__ __launch_bounds__(kNT) void k_cg_update_fold(int64_t n, const T* __re
 // IC(0) factor has the 5-point pattern, a whole batch of CG iterations runs
 // in one workgroup with no launch between the steps.  The factor (U's east
 // and north entries and the inverted diagonal) and the sweep vector stay in
-// LDS; x, r and p stay in registers (rows tid, tid + 512, ...).  One
-// wavefront runs both sweeps with lane j on grid line j: at step s it
-// finishes cell i = s - j, whose two dependencies are its own previous result
+// LDS; seven wavefronts own the rows and keep their x, r, p and entries of A in
+// registers from one iteration to the next.  The other wavefront runs both
+// sweeps with lane j on grid line j: at step s it finishes cell i = s - j, whose
+// two dependencies are its own previous result
 // (the cell before it on the line) and lane j-1's previous one, passed by a
 // DPP lane shift -- a step is the dependent arithmetic of the row and no
 // memory round trip.  Each row applies its entries in the order of the
@@ -370,8 +371,10 @@ __global__ __launch_bounds__(kNT) void k_cg_update_fold(int64_t n, const T* __re
 // test and history follow the multi-kernel CG (cg.hpp:75-112); only the
 // order in which the dots are summed differs.
 constexpr int kGridNT = 512;
-constexpr int kGridRows = 8;   // rows per thread
-constexpr int64_t kGridMaxN = int64_t(kGridNT) * kGridRows;
+constexpr int kGridOwners = kGridNT - kWave;   // threads that own rows: all but the sweeping wavefront's
+constexpr int kGridRows = 10;                  // rows per thread
+constexpr int64_t kGridMaxN = 4096;
+static_assert(kGridMaxN <= int64_t(kGridOwners) * kGridRows, "every row has an owner");
 
 struct GridCgArgs {
     int32_t n, nx, ny, iters;
@@ -384,10 +387,19 @@ struct GridCgArgs {
     KState* st;
 };
 
-// LDS doubles of the kernel: 8 of slack, sweep vector, east (one leading 0),
-// north (nx leading 0s), inverted diagonal, one dump slot per lane, 8 zeros.
-constexpr int kGridSlack = 8;
-inline int64_t grid_cg_lds_doubles(int64_t n, int64_t nx) { return kGridSlack + 4 * n + nx + 1 + kWave + 8; }
+// LDS layout: four arrays (sweep vector V, east, north, inverted diagonal) of
+// one pitch: grid line j's cells at pitch * j + kGridPad, its pads before them
+// and nine slots after the last line zero.  A turn of a line that has not begun
+// or has ended works on the zeros from `none`.
+constexpr int kGridPad = 8;
+struct GridLds {
+    int pitch, none, size;
+    __host__ __device__ GridLds(int64_t nx, int64_t ny)
+        : pitch(int(nx) + kGridPad), none(pitch * int(ny) + 1), size(none + kGridPad)
+    {
+    }
+};
+inline int64_t grid_cg_lds_doubles(int64_t nx, int64_t ny) { return 4 * int64_t(GridLds(nx, ny).size); }
 
 // Lane l receives lane l-1's value (lane 0: +0); lane l receives lane l+1's
 // (lane 63: +0).  DPP wave_shr:1 / wave_shl:1 on the two halves, lanes
@@ -414,203 +426,209 @@ __device__ inline double lane_from_next(double v)
 // the first operand from lane j-1, the second the lane's own last result.
 // Upper sweep on U, steps backwards (upper_trisolve.hpp:159-176):
 //   z_r = ((t_r - U[r][r+1] z_{r+1}) - U[r][r+nx] z_{r+nx}) * dinv_r.
-// Eight steps a turn.  Lane j reads step s's operands at element
-// nx*j + s - j of each array, so a turn's are eight consecutive elements
-// from a per-lane pointer that moves by eight a turn; the steps run on
-// registers (the dependent chain is the row's arithmetic and one lane
-// shift), with the next turn's loads issued before them.  Steps outside a
-// lane's line read neighbouring lines or the slack around the arrays (at
-// most 7 elements before V and 6 past D): a step before the line starts
-// gives +0 (the value of a missing neighbour), a step after it ends gives a
-// value no lane reads, and neither is stored (the dump slot takes it).
-// Lanes past the last line read eight zeros Z and give +0.  The step count
-// is rounded up to a multiple of eight.
-constexpr int kSweepTurn = 8;
+// Eight steps a turn, on eight consecutive elements of each array; the steps
+// run on registers, with the next turn's loads issued before them.
+// A lone wavefront's pace is its number of instructions (about 7 cycles each),
+// so nothing in a step looks at the line's ends: a step before its line
+// begins or after it ends meets a pad, zeros in every array, gives +0 (the value
+// of a missing neighbour) and stores +0 back.  Only whole turns outside the
+// line choose another address (`none`; lanes past the last line stay there).
+// With selects for the value and the address of each step instead, a step of a
+// 64 x 64 grid took 145 cycles; now 95.
+constexpr int kSweepTurn = kGridPad;
 
 template <bool LOWER>
-__device__ inline void grid_sweep(double* V, const double* E, const double* N, const double* D, double* dump,
-                                  const double* Z, int nx, int ny, int j)
+__device__ inline void grid_sweep(double* V, const double* E, const double* N, const double* D, const GridLds& G,
+                                  int nx, int ny, int j)
 {
     const int steps = nx + ny - 1;
     const int turns = (steps + kSweepTurn - 1) / kSweepTurn;
-    const bool line = j < ny;
-    const int S = steps - 1;
-    // element of step s: nx*j + s - j; lower s = 8k + u, upper s = S - 8k - u
-    const int q0 = LOWER ? nx * j - j : nx * j - j + S - (kSweepTurn - 1);
-    const int stride = line ? (LOWER ? kSweepTurn : -kSweepTurn) : 0;
-    const double* pv = line ? V + q0 : Z;
-    const double* pf1 = line ? (LOWER ? N + q0 : E + 1 + q0) : Z;   // U[r-nx][r] / U[r][r+1]
-    const double* pf2 = line ? (LOWER ? E + q0 : N + nx + q0) : Z;  // U[r-1][r]  / U[r][r+nx]
-    const double* pd = line ? D + q0 : Z;
+    const int base = G.pitch * j + kGridPad;
+    // lowest cell of turn 0; lanes past the last line never come to one of theirs
+    const int first = j < ny ? (LOWER ? -j : steps - kSweepTurn - j) : LOWER ? -(1 << 28) : 1 << 28;
     double y = 0.0;   // the lane's last result
-    auto load = [&](int k, double (&v)[kSweepTurn], double (&f1)[kSweepTurn], double (&f2)[kSweepTurn],
+    auto at = [&](int k) {
+        const int i = LOWER ? first + kSweepTurn * k : first - kSweepTurn * k;
+        return unsigned(i + kSweepTurn - 1) < unsigned(nx + kSweepTurn - 1) ? base + i : G.none;
+    };
+    auto load = [&](int o, double (&v)[kSweepTurn], double (&f1)[kSweepTurn], double (&f2)[kSweepTurn],
                     double (&d)[kSweepTurn]) {
-        const int o = k * stride;
+        // U[r-nx][r] and U[r-1][r], or U[r][r+1] and U[r][r+nx]
+        const double* p1 = LOWER ? N + (j == 0 || o == G.none ? G.none : o - G.pitch) : E + o;
+        const double* p2 = LOWER ? E - 1 + o : N + o;
 #pragma unroll
         for (int u = 0; u < kSweepTurn; u++) {
-            const int e = o + (LOWER ? u : kSweepTurn - 1 - u);
-            v[u] = pv[e];
-            f1[u] = pf1[e];
-            f2[u] = pf2[e];
-            d[u] = pd[e];
+            const int e = LOWER ? u : kSweepTurn - 1 - u;
+            v[u] = V[o + e];
+            f1[u] = p1[e];
+            f2[u] = p2[e];
+            d[u] = D[o + e];
         }
     };
-    auto run = [&](int k, const double (&v)[kSweepTurn], const double (&f1)[kSweepTurn],
+    auto run = [&](int o, const double (&v)[kSweepTurn], const double (&f1)[kSweepTurn],
                    const double (&f2)[kSweepTurn], const double (&d)[kSweepTurn]) {
-        const int o = k * stride;
-        const int i0 = LOWER ? kSweepTurn * k - j : S - kSweepTurn * k - j;   // cell of step 0
 #pragma unroll
         for (int u = 0; u < kSweepTurn; u++) {
-            const int i = LOWER ? i0 + u : i0 - u;
             const double nb = LOWER ? lane_from_prev(y) : lane_from_next(y);
             double acc = LOWER ? v[u] - f1[u] * nb : v[u] - f1[u] * y;
             acc = LOWER ? acc - f2[u] * y : acc - f2[u] * nb;
-            const double yn = acc * d[u];
-            y = (LOWER ? i < 0 : i >= nx) ? 0.0 : yn;
-            double* at = line && i >= 0 && i < nx ? V + (q0 + o + (LOWER ? u : kSweepTurn - 1 - u)) : dump + j;
-            *at = y;
+            y = acc * d[u];
+            V[o + (LOWER ? u : kSweepTurn - 1 - u)] = y;
         }
     };
     // the next turn's operands are loaded before a turn's steps (two register
     // sets, no copies)
     double cv[kSweepTurn], c1[kSweepTurn], c2[kSweepTurn], cd[kSweepTurn];
     double nv[kSweepTurn], n1[kSweepTurn], n2[kSweepTurn], nd[kSweepTurn];
-    load(0, cv, c1, c2, cd);
+    int oc = at(0), on;
+    load(oc, cv, c1, c2, cd);
     for (int k = 0; k < turns; k += 2) {
-        if (k + 1 < turns) load(k + 1, nv, n1, n2, nd);
-        run(k, cv, c1, c2, cd);
+        on = at(k + 1);   // (a turn past the last one loads zeros)
+        load(on, nv, n1, n2, nd);
+        run(oc, cv, c1, c2, cd);
         if (k + 1 >= turns) break;
-        if (k + 2 < turns) load(k + 2, cv, c1, c2, cd);
-        run(k + 1, nv, n1, n2, nd);
+        oc = at(k + 2);
+        load(oc, cv, c1, c2, cd);
+        run(on, nv, n1, n2, nd);
     }
 }
 
-// Sum over the workgroup in a fixed order; every thread gets the total.
-__device__ inline double grid_cg_sum(double v, double* red)
+// Sum over the row owners in a fixed order; every owner gets the total.  All
+// wavefronts pass the barrier.  Each of an iteration's sums has its own red, so
+// none waits for the one before to be read.
+constexpr int kGridOwnerWaves = kGridOwners / kWave;
+__device__ inline double grid_cg_sum(double v, double* red, int wave)
 {
     v = wave_sum(v);
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    if (lane == 0) red[wave] = v;
+    if (threadIdx.x % kWave == 0) red[wave] = v;
     lds_barrier();
     double t = 0.0;
 #pragma unroll
-    for (int w = 0; w < kGridNT / kWave; w++) t += red[w];
-    lds_barrier();   // red is reused by the next sum
+    for (int w = 0; w < kGridOwnerWaves; w++) t += red[w];
     return t;
 }
 
+// Bound by the sweeps' chain of nx + ny - 1 steps each way.  A solve of a 64 x 64
+// grid took 25.7 us an iteration while all eight wavefronts owned rows and read
+// A again each time (sweeps 15 us, A's entries after them 4.8 us, A p row by row
+// 2.4 us), and takes 13.9 us now (sweeps 10 us).  Owners' rows in straight-line code
+// without a branch around a load, so that their LDS reads are in flight together.
 __global__ __launch_bounds__(kGridNT) void k_cg_ic0_grid(GridCgArgs a)
 {
     extern __shared__ double lds[];
-    __shared__ double red[kGridNT / kWave];
+    __shared__ double red[3][kGridOwnerWaves];
     __shared__ KState ks;
     const int n = a.n, nx = a.nx, tid = threadIdx.x;
-    double* V = lds + kGridSlack;
-    double* E = V + n;        // E[1 + r] = U[r][r+1]
-    double* N = E + n + 1;    // N[nx + r] = U[r][r+nx]
-    double* D = N + n + nx;
-    double* dump = D + n;
-    double* Z = dump + kWave;   // eight zeros
-    for (int k = tid; k < n; k += kGridNT) {
-        E[1 + k] = a.east[k];
-        N[nx + k] = a.north[k];
-        D[k] = a.dinv[k];
-    }
-    if (tid == 0) E[0] = 0.0;
-    for (int k = tid; k < nx; k += kGridNT) N[k] = 0.0;
-    if (tid < kGridSlack) lds[tid] = 0.0;
-    if (tid < 8) Z[tid] = 0.0;
+    const GridLds G(nx, a.ny);
+    double* V = lds;
+    double* E = V + G.size;   // U[r][r+1]
+    double* N = E + G.size;   // U[r][r+nx]
+    double* D = N + G.size;
+    for (int k = tid; k < 4 * G.size; k += kGridNT) lds[k] = 0.0;
     if (tid == 0) ks = *a.st;
+    lds_barrier();
+    if (__builtin_amdgcn_readfirstlane(tid / kWave) == kGridOwnerWaves) {
+        // ---- the sweeping wavefront ----
+        __builtin_amdgcn_s_setprio(3);
+        lds_barrier();   // the factor and the state are in place
+        for (int it = 0; it < a.iters && !ks.done; it++) {
+            lds_barrier();   // r is in V
+            grid_sweep<true>(V, E, N, D, G, nx, a.ny, tid % kWave);
+            grid_sweep<false>(V, E, N, D, G, nx, a.ny, tid % kWave);
+            lds_barrier();   // z is in V
+            lds_barrier();   // (rho)
+            lds_barrier();   // (p is in V)
+            lds_barrier();   // (dot(p, q))
+            lds_barrier();   // (dot(r, r))
+            lds_barrier();   // (state)
+        }
+        return;
+    }
+    // ---- the row owners: rows tid, tid + kGridOwners, ... ----
+    const int wave = tid / kWave;
     double x[kGridRows], r[kGridRows], p[kGridRows], q[kGridRows];
-    int gi[kGridRows], gj[kGridRows], ge[kGridRows];   // grid position and first entry of each row
+    // A's entries: south (r-nx), west, centre, east, north (r+nx), 0 where the
+    // grid has no such neighbour
+    double cs[kGridRows], cw[kGridRows], cc[kGridRows], ce[kGridRows], cn[kGridRows];
+    int pos[kGridRows];   // place in the LDS arrays
+    auto in = [&](int u) { return tid + u * kGridOwners < n; };
 #pragma unroll
     for (int u = 0; u < kGridRows; u++) {
-        const int row = tid + u * kGridNT;
-        const bool in = row < n;
-        x[u] = in ? a.x[row] : 0.0;
-        r[u] = in ? a.r[row] : 0.0;
-        p[u] = in ? a.p[row] : 0.0;
-        gi[u] = in ? row % nx : 0;
-        gj[u] = in ? row / nx : 0;
-        ge[u] = in ? a.S[row] : 0;
+        const int row = tid + u * kGridOwners;
+        const int j = row / nx, i = row - j * nx;
+        x[u] = r[u] = p[u] = 0.0;
+        cs[u] = cw[u] = cc[u] = ce[u] = cn[u] = 0.0;
+        pos[u] = G.none;
+        if (in(u)) {
+            x[u] = a.x[row];
+            r[u] = a.r[row];
+            p[u] = a.p[row];
+            pos[u] = G.pitch * j + kGridPad + i;
+            E[pos[u]] = a.east[row];
+            N[pos[u]] = a.north[row];
+            D[pos[u]] = a.dinv[row];
+            int e = a.S[row];
+            if (j > 0) cs[u] = a.A[e++];
+            if (i > 0) cw[u] = a.A[e++];
+            cc[u] = a.A[e++];
+            if (i < nx - 1) ce[u] = a.A[e++];
+            if (j < a.ny - 1) cn[u] = a.A[e];
+        }
     }
     lds_barrier();
     for (int it = 0; it < a.iters && !ks.done; it++) {
         // z = solve(P, r)   (cg.hpp:97)
 #pragma unroll
         for (int u = 0; u < kGridRows; u++)
-            if (tid + u * kGridNT < n) V[tid + u * kGridNT] = r[u];
+            if (in(u)) V[pos[u]] = r[u];
         lds_barrier();
-        if (tid < kWave) {
-            grid_sweep<true>(V, E, N, D, dump, Z, nx, a.ny, tid);
-            grid_sweep<false>(V, E, N, D, dump, Z, nx, a.ny, tid);
-        }
-        lds_barrier();
-        // A's entries for q = A p, loaded now so they arrive while rho and p
-        // are formed: south (r-nx), west, centre, east, north (r+nx), 0 where
-        // the grid has no such neighbour
-        double cs[kGridRows], cw[kGridRows], cc[kGridRows], ce[kGridRows], cn[kGridRows];
-#pragma unroll
-        for (int u = 0; u < kGridRows; u++) {
-            const int row = tid + u * kGridNT;
-            const bool in = row < n, hs = in && gj[u] > 0, hw = in && gi[u] > 0, he = in && gi[u] < nx - 1,
-                       hn = in && gj[u] < a.ny - 1;
-            const int es = ge[u], ew = es + hs, ec = ew + hw, ee = ec + 1, en = ee + he;
-            cs[u] = hs ? a.A[es] : 0.0;
-            cw[u] = hw ? a.A[ew] : 0.0;
-            cc[u] = in ? a.A[ec] : 0.0;
-            ce[u] = he ? a.A[ee] : 0.0;
-            cn[u] = hn ? a.A[en] : 0.0;
-        }
-        // rho = dot(r, z)
+        lds_barrier();   // the sweeps
+        // rho = dot(r, z)   (rows past the last: 0 * 0)
+        double z[kGridRows];
         double acc = 0.0;
 #pragma unroll
-        for (int u = 0; u < kGridRows; u++)
-            if (tid + u * kGridNT < n) acc += r[u] * V[tid + u * kGridNT];
-        const double rho = grid_cg_sum(acc, red);
+        for (int u = 0; u < kGridRows; u++) {
+            z[u] = V[pos[u]];
+            acc += r[u] * z[u];
+        }
+        const double rho = grid_cg_sum(acc, red[0], wave);
         // p = z (first) or z + (rho / rho_1) p   (cg.hpp:99-102)
         const bool first = ks.i <= 1;
         const double beta = first ? 0.0 : rho / ks.rho_1;
 #pragma unroll
         for (int u = 0; u < kGridRows; u++) {
-            const int row = tid + u * kGridNT;
-            if (row < n) {
-                const double z = V[row];
-                p[u] = first ? z : z + beta * p[u];
-                V[row] = p[u];
+            if (in(u)) {
+                p[u] = first ? z[u] : z[u] + beta * p[u];
+                V[pos[u]] = p[u];
             }
         }
         lds_barrier();
-        // q = A p; alpha = rho / dot(p, q)   (cg.hpp:104-105)
+        // q = A p; alpha = rho / dot(p, q)   (cg.hpp:104-105): the row's
+        // entries in stored order (mat_vec_mult.hpp:662-687), a missing
+        // neighbour as 0 times a pad's 0
         acc = 0.0;
 #pragma unroll
         for (int u = 0; u < kGridRows; u++) {
-            const int row = tid + u * kGridNT;
-            q[u] = 0.0;
-            if (row < n) {   // the row's entries in stored order (mat_vec_mult.hpp:662-687)
-                double sum = 0.0;
-                if (gj[u] > 0) sum += cs[u] * V[row - nx];
-                if (gi[u] > 0) sum += cw[u] * V[row - 1];
-                sum += cc[u] * V[row];
-                if (gi[u] < nx - 1) sum += ce[u] * V[row + 1];
-                if (gj[u] < a.ny - 1) sum += cn[u] * V[row + nx];
-                q[u] = sum;
-                acc += p[u] * sum;
-            }
+            double sum = 0.0;
+            sum += cs[u] * V[max(pos[u] - G.pitch, 0)];   // (the line below the first: slot 0, a pad)
+            sum += cw[u] * V[pos[u] - 1];
+            sum += cc[u] * p[u];
+            sum += ce[u] * V[pos[u] + 1];
+            sum += cn[u] * V[min(pos[u] + G.pitch, G.none)];
+            q[u] = sum;
+            acc += p[u] * sum;
         }
-        const double alpha_1 = grid_cg_sum(acc, red);
+        const double alpha_1 = grid_cg_sum(acc, red[1], wave);
         const double alpha = rho / alpha_1;
         // x += alpha p; r -= alpha q; rr = dot(r, r)   (cg.hpp:107-109)
         acc = 0.0;
 #pragma unroll
-        for (int u = 0; u < kGridRows; u++)
-            if (tid + u * kGridNT < n) {
-                x[u] = x[u] + alpha * p[u];
-                const double ri = r[u] - alpha * q[u];
-                r[u] = ri;
-                acc += ri * ri;
-            }
-        const double rr = grid_cg_sum(acc, red);
+        for (int u = 0; u < kGridRows; u++) {
+            x[u] = x[u] + alpha * p[u];
+            r[u] = in(u) ? r[u] - alpha * q[u] : 0.0;
+            acc += r[u] * r[u];
+        }
+        const double rr = grid_cg_sum(acc, red[2], wave);
         if (tid == 0) {   // on a private copy: the shared one is written with LDS stores only
             KState t = ks;
             t.rho = rho;
@@ -625,8 +643,8 @@ __global__ __launch_bounds__(kGridNT) void k_cg_ic0_grid(GridCgArgs a)
     }
 #pragma unroll
     for (int u = 0; u < kGridRows; u++) {
-        const int row = tid + u * kGridNT;
-        if (row < n) {
+        const int row = tid + u * kGridOwners;
+        if (in(u)) {
             a.x[row] = x[u];
             a.r[row] = r[u];
             a.p[row] = p[u];
@@ -1185,8 +1203,9 @@ static int cg_t(m4g_matrix_s& A, void* xp, const void* bp, m4g_pc_s* P, m4g_iter
         DevBuf<double> east, north, dinv;
         const char* env = std::getenv("M4G_GRID_CG");   // M4G_GRID_CG=0: the multi-kernel path
         const bool enabled = !(env && std::atoi(env) == 0);
-        const size_t lds = P && enabled ? size_t(grid_cg_lds_doubles(n, P->grid.nx)) * sizeof(double) : 0;
-        if (P && enabled && lds <= grid_cg_lds_limit() && grid5_pattern(A, P->grid) &&
+        const bool small = P && enabled && n <= kGridMaxN;
+        const size_t lds = small ? size_t(grid_cg_lds_doubles(P->grid.nx, P->grid.ny)) * sizeof(double) : 0;
+        if (small && lds <= grid_cg_lds_limit() && grid5_pattern(A, P->grid) &&
             pc_grid_factor(*P, kGridMaxN, east, north, dinv, st)) {
             grid = true;
             static size_t granted = 0;

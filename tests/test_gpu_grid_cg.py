@@ -184,3 +184,23 @@ def test_rho_from_the_last_sweep(g, case, monkeypatch):
     np.testing.assert_allclose(fused[3][:k], separate[3][:k], rtol=1e-7)
     ref = o.solve("cg", A, b, pc=o.PC_IC0 if kind == g.PC_IC0 else o.PC_ILU0, max_iter=3000, rtol=1e-10)
     assert abs(fused[1] - ref["iterations"]) <= 1
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 64), (63, 64), (2, 64), (3, 2), (7, 9), (8, 8), (9, 7), (1000, 4), (2048, 2),
+                                   (45, 10), (64, 7)])
+def test_grid_cg_at_the_edges_of_its_turns_and_owners(g, nx, ny, monkeypatch):
+    # lines shorter than a turn, exact turns and one past them, one to all rows of an owner in use;
+    # against the multi-kernel solve, whose sums differ in their order only
+    S, I, V = g.varcoef5(nx, ny, seed=nx)
+    n = len(S) - 1
+    b = o.spmv(o.CSR(S, I, V), g.rng_uniform(4, 1, n))
+    rtol = 1e-8
+    say(f"  grid {nx} x {ny}")
+    got = solve(g, S, I, V, b, rtol)
+    monkeypatch.setenv("M4G_GRID_CG", "0")
+    multi = solve(g, S, I, V, b, rtol)
+    assert got["status"] == multi["status"] == o.OK
+    assert abs(got["iterations"] - multi["iterations"]) <= 1
+    k = min(len(got["history"]), len(multi["history"]), 20)
+    np.testing.assert_allclose(got["history"][:k], multi["history"][:k], rtol=1e-8, atol=1e-13 * o.two_norm(b))
+    assert np.max(np.abs(got["x"] - multi["x"])) <= 1e-6 * max(1.0, np.max(np.abs(multi["x"])))
