@@ -325,8 +325,8 @@ __device__ inline int sweep_role(const int* simd, int wave)
 // set by LDS and arithmetic latency only.  A sweep is bound by its chain of
 // dependent steps and of hand-overs between tiles, not by bytes.  Eight
 // wavefronts with the roles placed by SIMD and three polls in flight, against
-// five wavefronts in fixed roles with one poll at a time (two IC(0)/ILU(0) sweeps
-// in double, median of one): 7-point grid of 128^3 140.7 -> 128.3 us, 27-point
+// five wavefronts in fixed roles with one poll at a time (one IC(0) or ILU(0) sweep
+// in double, median): 7-point grid of 128^3 140.7 -> 128.3 us, 27-point
 // grid of 96^3 315.8 -> 284.4 us (with rows in one piece of 13, see
 // sweep_piece_width), a mesh of 64 400 vertices 174.3 -> 174.9 us.
 template <typename FV, typename VT, bool UNIT, int W>
