@@ -493,13 +493,42 @@ __device__ inline void grid_sweep(double* V, const double* E, const double* N, c
     }
 }
 
+// Sum over a wavefront in a fixed order, in every lane: within rows of 16 lanes by
+// DPP (neighbour, pair, half row, row mirrored), then the four rows' sums.  Three
+// a CG iteration, with nothing beside them:
+// 13.9 us an iteration with lane permutes through LDS, 13.5 us so (64 x 64).
+template <int CTRL>
+__device__ inline double dpp_add(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp(int(b), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(int(b >> 32), CTRL, 0xF, 0xF, true);
+    return v + __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+__device__ inline double grid_wave_sum(double v)
+{
+    v = dpp_add<0xB1>(v);    // quad_perm 1,0,3,2
+    v = dpp_add<0x4E>(v);    // quad_perm 2,3,0,1
+    v = dpp_add<0x141>(v);   // row_half_mirror
+    v = dpp_add<0x140>(v);   // row_mirror
+    const long long b = __double_as_longlong(v);
+    double t[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int lo = __builtin_amdgcn_readlane(int(b), 16 * k), hi = __builtin_amdgcn_readlane(int(b >> 32), 16 * k);
+        t[k] = __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+    }
+    return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
 // Sum over the row owners in a fixed order; every owner gets the total.  All
 // wavefronts pass the barrier.  Each of an iteration's sums has its own red, so
 // none waits for the one before to be read.
 constexpr int kGridOwnerWaves = kGridOwners / kWave;
 __device__ inline double grid_cg_sum(double v, double* red, int wave)
 {
-    v = wave_sum(v);
+    v = grid_wave_sum(v);
     if (threadIdx.x % kWave == 0) red[wave] = v;
     lds_barrier();
     double t = 0.0;
@@ -511,7 +540,7 @@ __device__ inline double grid_cg_sum(double v, double* red, int wave)
 // Bound by the sweeps' chain of nx + ny - 1 steps each way.  A solve of a 64 x 64
 // grid took 25.7 us an iteration while all eight wavefronts owned rows and read
 // A again each time (sweeps 15 us, A's entries after them 4.8 us, A p row by row
-// 2.4 us), and takes 13.9 us now (sweeps 10 us).  Owners' rows in straight-line code
+// 2.4 us), and takes 13.5 us now (sweeps 10 us).  Owners' rows in straight-line code
 // without a branch around a load, so that their LDS reads are in flight together.
 __global__ __launch_bounds__(kGridNT) void k_cg_ic0_grid(GridCgArgs a)
 {
