@@ -216,6 +216,12 @@ struct LineArgs {
 // by ticket, so every wait is for a workgroup that has started or for another
 // role of the same one.
 //
+// The partials of dot(w, y) are formed by the loader.  A lane of it meets about
+// one cell for every step of its strip, far more than a thread of the general
+// sweep does (26 at most), so products are added up in double whatever the
+// vectors' type is, eight sums of one level to one of the next (DotSum): the
+// longest chain of additions stays as short.
+//
 // The compute wavefront's pace is its number of instructions (about 7 cycles
 // each, alone on its SIMD), so it does nothing else and shares its SIMD with no
 // polling loop.  The hardware spreads the eight wavefronts evenly over the
@@ -243,6 +249,23 @@ struct alignas(16) LineFlags {
     int stored;     // blocks of results taken by the storer, and a ring's
     int exported;   // blocks of results taken by the exporter, and a ring's
     int finished;   // blocks the compute wavefront has finished
+};
+
+struct DotSum {
+    double level[4] = {0, 0, 0, 0};
+    __device__ void add(double block, int b)   // the sum of block b's products; b from 0 up
+    {
+        level[0] += block;
+        if ((b & 7) == 7) carry(0);
+        if ((b & 63) == 63) carry(1);
+        if ((b & 511) == 511) carry(2);
+    }
+    __device__ void carry(int k)
+    {
+        level[k + 1] += level[k];
+        level[k] = 0;
+    }
+    __device__ double total() const { return ((level[0] + level[1]) + level[2]) + level[3]; }
 };
 
 template <typename FV, typename VT, bool UNIT, bool FAR_FIRST>
@@ -412,7 +435,7 @@ __global__ __launch_bounds__(kLineWaves * kWave) void k_line_sweep(LineArgs a, c
                 __builtin_amdgcn_sched_barrier(0);
             }
             lds_barrier();
-            VT acc = 0;
+            DotSum sum;
             // block b takes the place of block b - RB once that one is finished (and, for the dot, its results read)
             auto run = [&](auto with_dot) {
                 constexpr bool dot = decltype(with_dot)::value;
@@ -424,9 +447,13 @@ __global__ __launch_bounds__(kLineWaves * kWave) void k_line_sweep(LineArgs a, c
                             wait_finished(d);
                             if constexpr (dot) {
                                 const VT* p = yring + (d * B & (kLineRing - 1));
+                                double t[8];   // (a cell outside the grid may hold anything)
 #pragma unroll
-                                for (int q = 0; q < 8; q++)
-                                    if (offset(q, d) != kNoCell) acc += wbuf[f][q] * p[8 * q * kLineRow];
+                                for (int q = 0; q < 8; q++) {
+                                    const double prod = double(wbuf[f][q]) * double(p[8 * q * kLineRow]);
+                                    t[q] = offset(q, d) != kNoCell ? prod : 0.0;
+                                }
+                                sum.add(((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7])), d);
                             }
                         }
                         if (b < nb) {
@@ -443,7 +470,7 @@ __global__ __launch_bounds__(kLineWaves * kWave) void k_line_sweep(LineArgs a, c
             };
             if (dot_with) run(std::true_type());
             else run(std::false_type());
-            dacc = double(acc);
+            dacc = sum.total();
         } else {
             lds_barrier();
             const auto yres = buffer_of(y, bytes);

@@ -128,3 +128,27 @@ def test_a_wait_that_gave_up_is_reported_by_each_direction_and_cleared(g, monkey
             assert e.value.status == g.ERR_TIMEOUT
         for _ in range(2):
             np.testing.assert_array_equal(apply(g, P, v, adjoint=adjoint), ref)
+
+
+def test_partials_of_the_last_sweep_on_long_lines(g):
+    # A = I on a star pattern: alpha of the first CG step is r.z / r.r = 1.  The last cells of each line,
+    # which the upper sweep meets first, are 1, the others so small that a float sum that holds a few
+    # ones drops their squares: 15 000 of them, 8e-4 of the whole.  Both dots add few products (at most 52)
+    # in a row in float and the rest in double: alpha is off by 52 * 2**-24 = 3.1e-6 each at most.
+    nx, ny = 15000, 66
+    print(f"partials in float {nx} x {ny}", flush=True)
+    S, I, V = star(nx, ny, 1, seed=1)
+    V = np.where(I == np.repeat(np.arange(nx * ny), np.diff(S)), 1.0, 0.0)
+    small = np.float32(np.sqrt(0.45 * 2.0 ** -20))
+    b = np.full((ny, nx), small, np.float32)
+    b[:, -8:] = 1.0
+    Ag = g.Matrix(S, I, V)
+    P = g.PC(Ag, g.PC_IC0, np.float32)
+    assert P.stats()["tiles_upper"] == 2
+    x = g.Vector(nx * ny, dtype=np.float32)
+    x.fill(0.0)
+    it, _ = g.make_iteration(1, 1e-30, 0.0, float(np.linalg.norm(b.astype(np.float64))))
+    g.cg(Ag, x, g.Vector(data=b.ravel(), dtype=np.float32), P, it)
+    alpha = x.numpy()[nx - 1]
+    print(f"  alpha - 1 = {alpha - 1.0:.2e}", flush=True)
+    assert abs(alpha - 1.0) <= 1e-5
