@@ -204,7 +204,7 @@ struct LineArgs {
     unsigned* tickets;           // [0] next ticket, [1] finished strips
     int* fault;
     int64_t other_count;         // entries of the other direction's exchange buffer
-    int64_t spin_limit;
+    int64_t wait_ticks;          // bound of a wait (BoundedWait)
     double* dot_partials;        // [strips], or null
 };
 
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(kLineWaves * kWave) void k_line_sweep(LineArgs a, c
             const auto src = buffer_of(xbuf + int64_t(strip - 1) * S + lead, unsigned(count) * unsigned(sizeof(VT)));
             int head = 0, from[kPolls];
             VT val[kPolls];
-            int64_t polls = 0;
+            BoundedWait wait{a.wait_ticks, a.fault};
             auto poll = [&](int k) {   // (past the end: 0)
                 from[k] = head;
                 val[k] = buffer_load<VT, 0x10>(src, unsigned(head + lane) * unsigned(sizeof(VT)));
@@ -519,10 +519,9 @@ __global__ __launch_bounds__(kLineWaves * kWave) void k_line_sweep(LineArgs a, c
                         if (from[k] + lane < got) west[from[k] + lane] = val[k];
                         head = got;
                         publish();
+                        wait.progress();
                     } else if (head < count) {
-                        ++polls;
-                        if (polls > a.spin_limit || ((polls & 63) == 0 && __hip_atomic_load(a.fault, __ATOMIC_RELAXED,
-                                                                                           __HIP_MEMORY_SCOPE_AGENT))) {
+                        if (wait.over()) {
                             // give up: the host reports the fault, the results are meaningless
                             if (lane == 0) __hip_atomic_store(a.fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                             head = count;
@@ -662,7 +661,7 @@ static void launch_line_t(LineSweep& d, LineSweep& other, const LineArgs& a, con
     else launch_line<FV, VT, false, true>(d, other, a, v, y, skip, dot_with, s);
 }
 
-void LineSweep::launch(LineSweep& other, const void* v, void* y, int vtype, const int* skip, int64_t spin_limit,
+void LineSweep::launch(LineSweep& other, const void* v, void* y, int vtype, const int* skip, int64_t wait_ticks,
                        const void* dot_with, double* dot_partials, hipStream_t s)
 {
     LineArgs a;
@@ -671,7 +670,7 @@ void LineSweep::launch(LineSweep& other, const void* v, void* y, int vtype, cons
     a.tickets = tickets.ptr;
     a.fault = fault.ptr;
     a.other_count = other.exchange_count();
-    a.spin_limit = spin_limit;
+    a.wait_ticks = wait_ticks;
     a.dot_partials = dot_partials;
     if (factor_type == M4G_F64) launch_line_t<double, double>(*this, other, a, v, y, skip, dot_with, s);
     else if (vtype == M4G_F64) launch_line_t<float, double>(*this, other, a, v, y, skip, dot_with, s);

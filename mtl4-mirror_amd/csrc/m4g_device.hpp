@@ -21,6 +21,29 @@ __device__ inline void lds_barrier()
 // The SIMD (0..3) of its compute unit that a wavefront runs on.
 __device__ inline int simd_id() { return __builtin_amdgcn_s_getreg((1 << 11) | (4 << 6) | 4); }   // HW_ID, bits 5:4
 
+// A polling wavefront's bounded wait.  It is bounded by time, not by a count of
+// polls: how long a poll takes depends on how many are in flight (0.47 us with
+// one at a time, 0.24 and 0.12 us with three in the tile and the line sweeps).  Of the time
+// between two looks at the clock, eight polls apart, at most 100 us count: while
+// the wavefront is preempted, so is the one it waits for.
+constexpr int64_t kWaitTicksPerUs = 100;   // of wall_clock64
+struct BoundedWait {
+    int64_t limit;       // ticks a wait may last since the last value that arrived
+    const int* fault;    // set by a wavefront that gave up
+    int64_t waited = 0, last = 0, polls = 0;
+    __device__ void progress() { waited = polls = 0; }
+    // after a poll that found nothing new: true when it is time to give up
+    __device__ bool over()
+    {
+        if ((++polls & 7) != 0) return false;
+        const int64_t now = int64_t(wall_clock64());
+        if (polls > 8) waited += min(now - last, 100 * kWaitTicksPerUs);
+        last = now;
+        return waited > limit ||
+               ((polls & 63) == 0 && __hip_atomic_load(fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    }
+};
+
 // Butterfly sum over the 64 lanes of a wavefront; every lane gets the total.
 // The combination order is fixed, so results are deterministic.
 __device__ inline double wave_sum(double v)

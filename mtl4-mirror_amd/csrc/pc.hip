@@ -204,7 +204,7 @@ struct SweepArgs {
     unsigned* tickets;                // [0] next ticket, [1] finished tiles
     int* fault;                       // set when a bounded wait runs out
     int64_t other_nexport;            // size of the other direction's exchange buffer
-    int64_t spin_limit;
+    int64_t wait_ticks;               // bound of a wait (BoundedWait)
     const void* dot_with;             // w (vector type), or null: no dot
     double* dot_partials;             // [ntiles] per tile: sum of w_r * y_r over its rows
 };
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4
         // behind the compute wavefront's LDS traffic.
         const int32_t* slot_of = reinterpret_cast<const int32_t*>(imp);
         int head = 0;
-        int64_t polls = 0;
+        BoundedWait wait{a.wait_ticks, a.fault};
         int32_t xs[kImportDepth];   // exchange slot of import head + lane + 64u; -1: none
         auto read_slots = [&]() {
 #pragma unroll
@@ -509,10 +509,9 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
                     if (lane == 0) __hip_atomic_store(&progress, head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     read_slots();   // the values written above lie below head
+                    wait.progress();
                 } else if (head < ni) {
-                    ++polls;
-                    if (polls > a.spin_limit ||
-                        ((polls & 63) == 0 && __hip_atomic_load(a.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                    if (wait.over()) {
                         // give up: flag the fault and release the compute wavefront
                         // (its results are then meaningless; the host reports the fault)
                         head = ni;
@@ -903,12 +902,14 @@ void SweepDev::ensure_exchange(int vtype)
 }
 
 
-// Polls a sweep's bounded waits make before giving up (M4G_SPIN_LIMIT; read
-// at every launch, so a process can change it between solves).
-static int64_t spin_limit()
+// How long a sweep waits for a value before it gives up, in ticks: M4G_SPIN_LIMIT
+// polls of half a microsecond, 2^20 of them (0.52 s) by default.  Read at every launch,
+// so a process can change it between solves.
+static int64_t wait_ticks()
 {
     const char* e = std::getenv("M4G_SPIN_LIMIT");
-    return e ? std::max<int64_t>(1, std::atoll(e)) : int64_t(1) << 20;   // about one second
+    const int64_t polls = e ? std::max<int64_t>(1, std::atoll(e)) : int64_t(1) << 20;
+    return std::min<int64_t>(polls, int64_t(1) << 50) * (kWaitTicksPerUs / 2);
 }
 
 // Dynamic LDS of a sweep launch (layout in sweep_lds_layout).
@@ -968,7 +969,7 @@ static void launch_sweep_t(SweepDev& d, SweepDev& other, const VT* v, VT* y, con
     a.tickets = d.tickets.ptr;
     a.fault = d.fault.ptr;
     a.other_nexport = other.plan_meta.nexport;
-    a.spin_limit = spin_limit();
+    a.wait_ticks = wait_ticks();
     a.dot_with = dot_with;
     a.dot_partials = dot_partials;
     VT* xo = (VT*)other.xbuf.ptr;
@@ -1003,7 +1004,7 @@ void run_sweep_pair(SweepDev& first, SweepDev& second, const void* v, void* tmp,
             SweepDev& d = dir ? second : first;
             const SweepPlan& p = d.plan_meta;
             TraceRange tr(!p.lower ? kTraceUpperTrisolve : p.unit ? kTraceLowerUnitTrisolve : kTraceLowerTrisolve);
-            d.line->launch(dir ? *first.line : *second.line, dir ? tmp : v, dir ? y : tmp, vtype, skip, spin_limit(),
+            d.line->launch(dir ? *first.line : *second.line, dir ? tmp : v, dir ? y : tmp, vtype, skip, wait_ticks(),
                            dir ? dot_with : nullptr, dir ? dot_partials : nullptr, s);
         }
         return;

@@ -1,13 +1,14 @@
 """Failure handling forced from the host.
 
-A sweep's bounded waits give up after M4G_SPIN_LIMIT polls (read at every
-launch).  With a limit of one poll, the tiles of a multi-tile sweep give up
+A sweep's bounded waits give up after M4G_SPIN_LIMIT polls of half a microsecond
+(read at every launch).  With a limit of one poll, the tiles of a multi-tile sweep give up
 waiting for values their upstream tiles have not exported yet, every wave
 still runs to its end, and the call reports M4G_ERR_TIMEOUT.  The fault flag
 is cleared when it is reported, so later calls with the normal limit give the
 exact results again.  Also: the torch binding rejects tensors of a type the
 kernels do not read."""
 import os
+import time
 
 import numpy as np
 import pytest
@@ -63,6 +64,47 @@ def test_sweep_timeout_is_reported_then_cleared(g, monkeypatch):
     assert abs(it.iterations - ref_cg["iterations"]) <= max(1, int(np.ceil(0.02 * ref_cg["iterations"])))
     print(f"after the limit is restored: exact application, CG {it.iterations} it "
           f"(oracle {ref_cg['iterations']})", flush=True)
+
+
+def chain(n):
+    """Rows that each depend on the one before and on another not far back: one row a level, no grid."""
+    rng = np.random.default_rng(1)
+    r = np.arange(n)
+    far = np.maximum(r - 2 - rng.integers(0, 40, n), 0)
+    rows = np.concatenate([r, r[1:], r[3:], r[:-1], far[3:]])
+    cols = np.concatenate([r, r[:-1], far[3:], r[1:], r[3:]])
+    key = np.unique(rows * n + cols)
+    rows, cols = key // n, key % n
+    return np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]), cols, np.where(rows == cols, 4.0, -0.5)
+
+
+@pytest.mark.parametrize("form,polls", [("lines", 1000), ("tiles", 8000)])
+def test_a_wait_lasts_as_long_as_its_limit_says(g, form, polls, monkeypatch):
+    # both directions of an application wait for more than the limit, one after the other, and give up;
+    # with a limit of twice a sweep's own time none does
+    S, I, V = g.varcoef5(64, 16384, seed=1) if form == "lines" else chain(120000)
+    n = len(S) - 1
+    P = g.PC(g.Matrix(S, I, V), g.PC_ILU0)
+    x, y = g.Vector(data=g.rng_uniform(8, 1, n)), g.Vector(n)
+    P.solve(x, y)
+    ref = y.numpy()
+    t0 = time.perf_counter()
+    P.solve(x, y)
+    usual = time.perf_counter() - t0
+    print(f"{form}: {P.stats()['tiles_lower']} of {n} rows, an application takes {1e3 * usual:.2f} ms", flush=True)
+    limit = polls * 0.5e-6
+    monkeypatch.setenv("M4G_SPIN_LIMIT", str(polls))
+    for _ in range(2):   # (the process's first error costs more than the wait)
+        t0 = time.perf_counter()
+        with pytest.raises(g.M4GError) as e:
+            P.solve(x, y)
+        waited = time.perf_counter() - t0
+        print(f"  gave up after {1e3 * waited:.2f} ms, limit {1e3 * limit:.2f} ms a sweep", flush=True)
+        assert e.value.status == g.ERR_TIMEOUT
+        assert waited >= 2 * limit
+    monkeypatch.setenv("M4G_SPIN_LIMIT", str(int(usual / 0.5e-6)))
+    P.solve(x, y)
+    np.testing.assert_array_equal(y.numpy(), ref)
 
 
 def test_vector_rejects_unsupported_tensor_types(g):
