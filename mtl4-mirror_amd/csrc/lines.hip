@@ -69,6 +69,14 @@ __host__ __device__ inline LineLds line_lds(int steps, int vbytes)
     return l;
 }
 
+// A strip holds coefficients for the lanes' skew as well: 24 * steps / nx bytes a
+// row in double, 54 with nx = 64, 960 with nx = 2, where the general sweep's records take
+// 64.  More than that is given for the speed (2 x 50 000: 5.7 against 12.1 ms an
+// application) up to this size; a larger narrow grid takes the general sweep, so
+// that whatever fits the card with records fits.
+constexpr int64_t kLinePadBytes = int64_t(256) << 20;
+constexpr int64_t kRecordRowBytes = 64;
+
 LineGeom line_geometry(const GridInfo& g, size_t lds_budget)
 {
     LineGeom G;
@@ -76,10 +84,12 @@ LineGeom line_geometry(const GridInfo& g, size_t lds_budget)
     if (g.nz != 1 || g.nx < 2 || g.ny < 2 || g.nx * g.ny >= (int64_t(1) << 29) - 64) return G;
     const int64_t steps = (g.nx + 63 + 7 + kLineDepth - 1) / kLineDepth * kLineDepth;   // the lanes' skew and the phase
     if (steps >= (1 << 20) || line_lds(int(steps), 8).total > lds_budget) return G;
+    const int64_t strips = (g.ny + 63) / 64;
+    if (strips * steps * kWave * 24 > std::max(kLinePadBytes, g.nx * g.ny * kRecordRowBytes)) return G;
     G.nx = int32_t(g.nx);
     G.ny = int32_t(g.ny);
     G.steps = int32_t(steps);
-    G.strips = int32_t((g.ny + 63) / 64);
+    G.strips = int32_t(strips);
     return G;
 }
 

@@ -32,7 +32,8 @@ struct LineGeom {
     __host__ __device__ int32_t n() const { return nx * ny; }
 };
 
-// The geometry for a grid (strips 0 when it is not 2D or its lines are too long).
+// The geometry for a grid (strips 0 when it is not 2D, its lines are too long, or it is large and
+// so narrow that the coefficients would take more memory than the general sweep's records).
 LineGeom line_geometry(const GridInfo& g, size_t lds_budget);
 
 struct LineSweep {

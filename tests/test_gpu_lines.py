@@ -152,3 +152,19 @@ def test_partials_of_the_last_sweep_on_long_lines(g):
     alpha = x.numpy()[nx - 1]
     print(f"  alpha - 1 = {alpha - 1.0:.2e}", flush=True)
     assert abs(alpha - 1.0) <= 1e-5
+
+
+@pytest.mark.parametrize("nx,ny,lines", [(2, 139776, True), (2, 139777, False), (41, 128000, False), (42, 128000, True)])
+def test_large_narrow_grids_take_the_general_sweep(g, nx, ny, lines):
+    # above 256 MB of coefficients a strip may hold 64 bytes a row: 24 * (lanes and steps) / cells.
+    # nx = 2: 80 steps, 122 880 bytes a strip, 2184 strips at most; nx = 41 and 42: 112 steps, 65.6 and 64 bytes a row
+    print(f"narrow grid {nx} x {ny}", flush=True)
+    S, I, V = star(nx, ny, 1, seed=nx)
+    A = o.CSR(S, I, V)
+    v = g.rng_uniform(3, 1, A.n)
+    st, L, U = o.ilu0_factor(A)
+    P = g.PC(g.Matrix(S, I, V), g.PC_ILU0)
+    s = P.stats()
+    assert lines == (s["tiles_lower"] == -(-ny // 64) and s["tile_ny"] == 64), s
+    np.testing.assert_array_equal(apply(g, P, v), o.ilu0_solve(L, U, v))
+    np.testing.assert_array_equal(apply(g, P, v, adjoint=True), o.ilu0_adjoint_solve(L, U, v))
