@@ -168,3 +168,54 @@ def test_large_narrow_grids_take_the_general_sweep(g, nx, ny, lines):
     assert lines == (s["tiles_lower"] == -(-ny // 64) and s["tile_ny"] == 64), s
     np.testing.assert_array_equal(apply(g, P, v), o.ilu0_solve(L, U, v))
     np.testing.assert_array_equal(apply(g, P, v, adjoint=True), o.ilu0_adjoint_solve(L, U, v))
+
+
+@pytest.mark.parametrize("nx,ny", [(3722, 66), (3723, 66), (8000, 3), (16010, 3), (16011, 3)])
+def test_line_sweeps_on_the_longest_lines(g, nx, ny):
+    # a step holds 8 bytes of LDS: above 64 KB (nx = 3 723 on) it is asked for, above 160 KB (nx = 16 010) there
+    # is none and the general sweep takes the grid
+    print(f"long lines {nx} x {ny}", flush=True)
+    S, I, V = star(nx, ny, 1, seed=nx)
+    A = o.CSR(S, I, V)
+    v = g.rng_uniform(3, 1, A.n)
+    Ag = g.Matrix(S, I, V)
+    st, L, U = o.ilu0_factor(A)
+    P = g.PC(Ag, g.PC_ILU0)
+    s = P.stats()
+    assert (nx <= 16010) == (s["tiles_lower"] == -(-ny // 64) and s["tile_nx"] == nx and s["tile_ny"] == 64), s
+    np.testing.assert_array_equal(apply(g, P, v), o.ilu0_solve(L, U, v))
+    np.testing.assert_array_equal(apply(g, P, v, adjoint=True), o.ilu0_adjoint_solve(L, U, v))
+    st, Uc, Lc = o.ic0_factor(A)
+    P = g.PC(Ag, g.PC_IC0, np.float32)
+    np.testing.assert_array_equal(apply(g, P, v), o.ic0_solve(Lc, Uc, v, factor_dtype=np.float32))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("shape", [(2, 2, 1), (64, 65, 1), (700, 70, 1), (20, 33, 9)])
+def test_partials_of_the_last_sweep(g, shape, dtype, monkeypatch):
+    # alpha = r.z / p.Ap of the first CG step, from x = alpha z, against a dot kernel's: both add in double what
+    # float products and sums of at most 52 in a row give (52 * 2**-24 = 3.1e-6 for float), r.z > 0 without
+    # cancellation in the large
+    print(f"partials {shape} {np.dtype(dtype).name}", flush=True)
+    S, I, V = star(*shape, seed=3)
+    rows = np.repeat(np.arange(len(S) - 1), np.diff(S))
+    key = np.minimum(rows, I) * len(S) + np.maximum(rows, I)   # one value for both halves
+    off = rows != I
+    V[off] = -0.1 - (key[off] * 2654435761 % 1000) * 9e-4
+    b = 0.5 + g.rng_uniform(5, 1, len(S) - 1) ** 2
+    Ag = g.Matrix(S, I, V)
+    P = g.PC(Ag, g.PC_IC0, dtype)
+    z = apply(g, P, b.astype(dtype), dtype=dtype)
+    xs = []
+    for separate in (False, True):
+        if separate:
+            monkeypatch.setenv("M4G_CG_SWEEP_DOT", "0")
+        monkeypatch.setenv("M4G_GRID_CG", "0")
+        x = g.Vector(len(b), dtype=dtype)
+        x.fill(0.0)
+        it, _ = g.make_iteration(1, 1e-30, 0.0, 1.0)
+        g.cg(Ag, x, g.Vector(data=b, dtype=dtype), P, it)
+        xs.append(x.numpy())
+    k = np.argmax(z)
+    alpha = [float(x[k]) / float(z[k]) for x in xs]
+    assert abs(alpha[0] / alpha[1] - 1.0) <= (1e-13 if dtype == np.float64 else 1e-5), alpha
