@@ -1383,12 +1383,10 @@ int m4g_pc_create(m4g_pc* out, m4g_matrix A, int kind, int ftype)
             const GridInfo g = fg.get();
             mark("grid_wait");
             P->grid = g;
-            // the sweep plans need only the pattern: they are built on host
-            // threads while this thread runs the factorisation on the device
             // a 2D grid with the whole 5-point pattern: line sweeps, which need no plan (256 x 256: 30 us a sweep
-            // against 88; 64 x 64: 9 against 27).  They need a line's steps in LDS (line_geometry).
+            // against 88; 64 x 64: 9 against 27).  line_geometry names the limits.
             P->line = LineGeom();
-            if (g.nz == 1 && star_pattern(g, n, P->fS.data(), P->fI.data(), kind == M4G_PC_IC0))
+            if (star_pattern(g, n, P->fS.data(), P->fI.data(), kind == M4G_PC_IC0))
                 P->line = line_geometry(g, sweep_lds_budget());
             if (P->line.strips) {
                 factorize_levels(*P, lo, *A, lo_levels);
@@ -1402,6 +1400,8 @@ int m4g_pc_create(m4g_pc* out, m4g_matrix A, int kind, int ftype)
                 M4G_HIP(hipStreamSynchronize(s));   // `rows` is read by the copy
                 mark("lines");
             } else {
+                // the sweep plans need only the pattern: they are built on host
+                // threads while this thread runs the factorisation on the device
                 const int64_t cap = sweep_tile_cap(ftype == M4G_F64 ? M4G_F64 : M4G_F32);
                 PlanPairJob plans(lo, up, g, cap, ftype, &lo_levels);
                 factorize_levels(*P, lo, *A, lo_levels);

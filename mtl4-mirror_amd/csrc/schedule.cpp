@@ -250,22 +250,20 @@ GridInfo infer_grid(int64_t n, const int64_t* S, const int64_t* I)
 
 bool star_pattern(const GridInfo& g, int64_t n, const int64_t* S, const int64_t* I, bool upper_only)
 {
-    if (g.nx < 2 || g.ny < 2 || g.nx * g.ny * g.nz != n) return false;
-    const int64_t nx = g.nx, ny = g.ny, nxy = g.nx * g.ny;
+    if (g.nx < 2 || g.ny < 2 || g.nz != 1 || g.nx * g.ny != n) return false;
+    const int64_t nx = g.nx;
     int bad = 0;
     parallel_chunks(n, n >= 65536 ? plan_threads() : 1, [&](int64_t r0, int64_t r1, int) {
         for (int64_t r = r0; r < r1; r++) {
-            const int64_t i = r % nx, j = r / nx % ny;
-            int64_t want[7], m = 0;
+            const int64_t i = r % nx;
+            int64_t want[5], m = 0;
             if (!upper_only) {
-                if (r >= nxy) want[m++] = r - nxy;
-                if (j > 0) want[m++] = r - nx;
+                if (r >= nx) want[m++] = r - nx;
                 if (i > 0) want[m++] = r - 1;
             }
             want[m++] = r;
             if (i < nx - 1) want[m++] = r + 1;
-            if (j < ny - 1) want[m++] = r + nx;
-            if (r + nxy < n) want[m++] = r + nxy;
+            if (r + nx < n) want[m++] = r + nx;
             if (S[r + 1] - S[r] != m || !std::equal(want, want + m, I + S[r])) {
                 __atomic_store_n(&bad, 1, __ATOMIC_RELAXED);
                 return;

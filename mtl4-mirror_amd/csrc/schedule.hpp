@@ -60,8 +60,8 @@ struct GridInfo {
 };
 GridInfo infer_grid(int64_t n, const int64_t* starts, const int64_t* indices);
 
-// True when every row of the pattern holds exactly its in-grid neighbours of
-// the 5-point (nz == 1) or 7-point stencil and its diagonal, in column order;
+// True when the grid is 2D and every row of the pattern holds exactly its
+// in-grid neighbours of the 5-point stencil and its diagonal, in column order;
 // upper_only: the diagonal and the neighbours after it.
 bool star_pattern(const GridInfo& g, int64_t n, const int64_t* starts, const int64_t* indices, bool upper_only);
 
