@@ -431,8 +431,11 @@ __device__ inline double lane_from_next(double v)
 // A lone wavefront's pace is its number of instructions (about 7 cycles each),
 // so nothing in a step looks at the line's ends: a step before its line
 // begins or after it ends meets a pad, zeros in every array, gives +0 (the value
-// of a missing neighbour) and stores +0 back.  Only whole turns outside the
-// line choose another address (`none`; lanes past the last line stay there).
+// of a missing neighbour) and stores +0 back.  That holds while the values beside
+// the pad are finite; 0 * Inf leaves a NaN in it, for good.  By then rho = r.z and p.q
+// are not finite, so alpha is NaN and x, r and p are NaN in every row, as they
+// are without pads.  Only whole turns outside the line choose another address
+// (`none`; lanes past the last line stay there).
 // With selects for the value and the address of each step instead, a step of a
 // 64 x 64 grid took 145 cycles; now 95.
 constexpr int kSweepTurn = kGridPad;

@@ -204,3 +204,26 @@ def test_grid_cg_at_the_edges_of_its_turns_and_owners(g, nx, ny, monkeypatch):
     k = min(len(got["history"]), len(multi["history"]), 20)
     np.testing.assert_allclose(got["history"][:k], multi["history"][:k], rtol=1e-8, atol=1e-13 * o.two_norm(b))
     assert np.max(np.abs(got["x"] - multi["x"])) <= 1e-6 * max(1.0, np.max(np.abs(multi["x"])))
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 1e308])
+def test_grid_cg_with_values_that_are_not_finite(g, value, monkeypatch):
+    # (1e308: r is finite, its products overflow) the multi-kernel solve's outcome: no convergence, the same
+    # history, NaN in every row
+    S, I, V = g.varcoef5(20, 9, seed=2)
+    n = len(S) - 1
+    b = o.spmv(o.CSR(S, I, V), g.rng_uniform(4, 1, n))
+    b[77] = value
+    runs = []
+    for env in ("1", "0"):
+        monkeypatch.setenv("M4G_GRID_CG", env)
+        Ag = g.Matrix(S, I, V)
+        x = g.Vector(n)
+        x.fill(0.0)
+        it, hist = g.make_iteration(40, 1e-10, 0.0, 1.0)
+        st = g.cg(Ag, x, g.Vector(data=b), g.PC(Ag, g.PC_IC0), it)
+        runs.append((st, it.iterations, x.numpy(), hist))
+    say(f"  {value}: status {runs[0][0]}, {runs[0][1]} iterations, {np.isnan(runs[0][2]).sum()} of {n} NaN")
+    assert runs[0][:2] == runs[1][:2]
+    np.testing.assert_array_equal(runs[0][2], runs[1][2])
+    np.testing.assert_array_equal(runs[0][3], runs[1][3])
