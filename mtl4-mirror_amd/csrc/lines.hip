@@ -48,6 +48,7 @@ constexpr int kLineHeader = 128;    // bytes: counters of the workgroup
 constexpr int kLineZeros = 16;      // zeros read in place of imports by the first strip
 constexpr int kLineLead = 63;       // steps by which the strip before is ahead when it has the value a step needs
 constexpr int kLineWaves = 8;
+constexpr int kLinePollsPerSpin = 5;   // polls in half a microsecond and a little more (one takes 0.12 us, three in flight)
 constexpr int kDone = 1 << 30;
 
 // A strip's first line starts at step `line_phase`, chosen so that the imports
@@ -214,7 +215,7 @@ struct LineArgs {
     unsigned* tickets;           // [0] next ticket, [1] finished strips
     int* fault;
     int64_t other_count;         // entries of the other direction's exchange buffer
-    int64_t wait_ticks;          // bound of a wait (BoundedWait)
+    int64_t poll_limit;          // fruitless polls of a strip's importer
     double* dot_partials;        // [strips], or null
 };
 
@@ -509,7 +510,7 @@ __global__ __launch_bounds__(kLineWaves * kWave) void k_line_sweep(LineArgs a, c
             const auto src = buffer_of(xbuf + int64_t(strip - 1) * S + lead, unsigned(count) * unsigned(sizeof(VT)));
             int head = 0, from[kPolls];
             VT val[kPolls];
-            BoundedWait wait{a.wait_ticks, a.fault};
+            BoundedWait wait{a.poll_limit, a.fault};
             auto poll = [&](int k) {   // (past the end: 0)
                 from[k] = head;
                 val[k] = buffer_load<VT, 0x10>(src, unsigned(head + lane) * unsigned(sizeof(VT)));
@@ -529,7 +530,6 @@ __global__ __launch_bounds__(kLineWaves * kWave) void k_line_sweep(LineArgs a, c
                         if (from[k] + lane < got) west[from[k] + lane] = val[k];
                         head = got;
                         publish();
-                        wait.progress();
                     } else if (head < count) {
                         if (wait.over()) {
                             // give up: the host reports the fault, the results are meaningless
@@ -671,7 +671,7 @@ static void launch_line_t(LineSweep& d, LineSweep& other, const LineArgs& a, con
     else launch_line<FV, VT, false, true>(d, other, a, v, y, skip, dot_with, s);
 }
 
-void LineSweep::launch(LineSweep& other, const void* v, void* y, int vtype, const int* skip, int64_t wait_ticks,
+void LineSweep::launch(LineSweep& other, const void* v, void* y, int vtype, const int* skip, int64_t spin_limit,
                        const void* dot_with, double* dot_partials, hipStream_t s)
 {
     LineArgs a;
@@ -680,7 +680,7 @@ void LineSweep::launch(LineSweep& other, const void* v, void* y, int vtype, cons
     a.tickets = tickets.ptr;
     a.fault = fault.ptr;
     a.other_count = other.exchange_count();
-    a.wait_ticks = wait_ticks;
+    a.poll_limit = spin_limit * kLinePollsPerSpin;
     a.dot_partials = dot_partials;
     if (factor_type == M4G_F64) launch_line_t<double, double>(*this, other, a, v, y, skip, dot_with, s);
     else if (vtype == M4G_F64) launch_line_t<float, double>(*this, other, a, v, y, skip, dot_with, s);

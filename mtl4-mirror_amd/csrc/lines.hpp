@@ -52,7 +52,7 @@ struct LineSweep {
     void init(const LineGeom& g, int kind, int ftype, const double* f, const int32_t* rows);
     int64_t exchange_count() const { return int64_t(G.steps) * G.strips; }   // entries of xbuf
     void prepare(int vtype, hipStream_t s);
-    void launch(LineSweep& other, const void* v, void* y, int vtype, const int* skip, int64_t wait_ticks,
+    void launch(LineSweep& other, const void* v, void* y, int vtype, const int* skip, int64_t spin_limit,
                 const void* dot_with, double* dot_partials, hipStream_t s);
 };
 

@@ -204,7 +204,7 @@ struct SweepArgs {
     unsigned* tickets;                // [0] next ticket, [1] finished tiles
     int* fault;                       // set when a bounded wait runs out
     int64_t other_nexport;            // size of the other direction's exchange buffer
-    int64_t wait_ticks;               // bound of a wait (BoundedWait)
+    int64_t poll_limit;               // fruitless polls of a tile's importer
     const void* dot_with;             // w (vector type), or null: no dot
     double* dot_partials;             // [ntiles] per tile: sum of w_r * y_r over its rows
 };
@@ -215,6 +215,7 @@ constexpr int kSweepWaves = 8;
 constexpr int kSweepThreads = kSweepWaves * kWave;
 constexpr int kImportDepth = 2;       // imports each importer lane polls at a time
 constexpr int kImportPolls = 3;       // polls in flight
+constexpr int kPollsPerSpin = 3;      // polls in half a microsecond and a little more (one takes 0.24 us)
 constexpr int kFillUnroll = 16;       // row values each thread moves at once between HBM and LDS
 constexpr int kFillLists = 5;         // import and export list entries per thread in the first fill pass
 
@@ -466,7 +467,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4
         // behind the compute wavefront's LDS traffic.
         const int32_t* slot_of = reinterpret_cast<const int32_t*>(imp);
         int head = 0;
-        BoundedWait wait{a.wait_ticks, a.fault};
+        BoundedWait wait{a.poll_limit, a.fault};
         int32_t xs[kImportDepth];   // exchange slot of import head + lane + 64u; -1: none
         auto read_slots = [&]() {
 #pragma unroll
@@ -509,7 +510,6 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
                     if (lane == 0) __hip_atomic_store(&progress, head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     read_slots();   // the values written above lie below head
-                    wait.progress();
                 } else if (head < ni) {
                     if (wait.over()) {
                         // give up: flag the fault and release the compute wavefront
@@ -902,14 +902,15 @@ void SweepDev::ensure_exchange(int vtype)
 }
 
 
-// How long a sweep waits for a value before it gives up, in ticks: M4G_SPIN_LIMIT
-// polls of half a microsecond, 2^20 of them (0.52 s) by default.  Read at every launch,
-// so a process can change it between solves.
-static int64_t wait_ticks()
+// How long a sweep's wavefront waits for values, in all, before it gives up: M4G_SPIN_LIMIT
+// half microseconds at least, 2^20 of them by default.  Read at every launch, so a process
+// can change it between solves.  The kernels count polls, and how many of theirs make half a
+// microsecond depends on how many they have in flight (0.47 us a poll with one).
+static int64_t spin_limit()
 {
     const char* e = std::getenv("M4G_SPIN_LIMIT");
-    const int64_t polls = e ? std::max<int64_t>(1, std::atoll(e)) : int64_t(1) << 20;
-    return std::min<int64_t>(polls, int64_t(1) << 50) * (kWaitTicksPerUs / 2);
+    const int64_t limit = e ? std::max<int64_t>(1, std::atoll(e)) : int64_t(1) << 20;
+    return std::min<int64_t>(limit, int64_t(1) << 56);   // (it is multiplied)
 }
 
 // Dynamic LDS of a sweep launch (layout in sweep_lds_layout).
@@ -969,7 +970,7 @@ static void launch_sweep_t(SweepDev& d, SweepDev& other, const VT* v, VT* y, con
     a.tickets = d.tickets.ptr;
     a.fault = d.fault.ptr;
     a.other_nexport = other.plan_meta.nexport;
-    a.wait_ticks = wait_ticks();
+    a.poll_limit = spin_limit() * kPollsPerSpin;
     a.dot_with = dot_with;
     a.dot_partials = dot_partials;
     VT* xo = (VT*)other.xbuf.ptr;
@@ -1004,7 +1005,7 @@ void run_sweep_pair(SweepDev& first, SweepDev& second, const void* v, void* tmp,
             SweepDev& d = dir ? second : first;
             const SweepPlan& p = d.plan_meta;
             TraceRange tr(!p.lower ? kTraceUpperTrisolve : p.unit ? kTraceLowerUnitTrisolve : kTraceLowerTrisolve);
-            d.line->launch(dir ? *first.line : *second.line, dir ? tmp : v, dir ? y : tmp, vtype, skip, wait_ticks(),
+            d.line->launch(dir ? *first.line : *second.line, dir ? tmp : v, dir ? y : tmp, vtype, skip, spin_limit(),
                            dir ? dot_with : nullptr, dir ? dot_partials : nullptr, s);
         }
         return;

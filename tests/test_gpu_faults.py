@@ -1,7 +1,7 @@
 """Failure handling forced from the host.
 
-A sweep's bounded waits give up after M4G_SPIN_LIMIT polls of half a microsecond
-(read at every launch).  With a limit of one poll, the tiles of a multi-tile sweep give up
+A sweep's bounded waits give up after at least M4G_SPIN_LIMIT half microseconds
+(read at every launch).  With a limit of one, the tiles of a multi-tile sweep give up
 waiting for values their upstream tiles have not exported yet, every wave
 still runs to its end, and the call reports M4G_ERR_TIMEOUT.  The fault flag
 is cleared when it is reported, so later calls with the normal limit give the
@@ -78,8 +78,8 @@ def chain(n):
     return np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]), cols, np.where(rows == cols, 4.0, -0.5)
 
 
-@pytest.mark.parametrize("form,polls", [("lines", 1000), ("tiles", 8000)])
-def test_a_wait_lasts_as_long_as_its_limit_says(g, form, polls, monkeypatch):
+@pytest.mark.parametrize("form,spins", [("lines", 1000), ("tiles", 8000)])
+def test_a_wait_lasts_as_long_as_its_limit_says(g, form, spins, monkeypatch):
     # both directions of an application wait for more than the limit, one after the other, and give up;
     # with a limit of twice a sweep's own time none does
     S, I, V = g.varcoef5(64, 16384, seed=1) if form == "lines" else chain(120000)
@@ -92,8 +92,8 @@ def test_a_wait_lasts_as_long_as_its_limit_says(g, form, polls, monkeypatch):
     P.solve(x, y)
     usual = time.perf_counter() - t0
     print(f"{form}: {P.stats()['tiles_lower']} of {n} rows, an application takes {1e3 * usual:.2f} ms", flush=True)
-    limit = polls * 0.5e-6
-    monkeypatch.setenv("M4G_SPIN_LIMIT", str(polls))
+    limit = spins * 0.5e-6
+    monkeypatch.setenv("M4G_SPIN_LIMIT", str(spins))
     for _ in range(2):   # (the process's first error costs more than the wait)
         t0 = time.perf_counter()
         with pytest.raises(g.M4GError) as e:
