@@ -21,15 +21,19 @@
 //
 // What bounds it: the compute wavefront's instructions, 41 ns a step (18 ns of
 // them the dependent chain: lane shift and four FP64 operations) for nx + 63
-// steps a strip and about 3 us from strip to strip; HBM traffic (40 bytes a
-// row) is far below.  One wavefront per strip and workgroup, because two in one
-// workgroup slowed each other (60 against 78 ns a step).  Per sweep in double,
-// against the general sweep's tiles: 256 x 256 30 us (88), 301 x 173 28 us (80),
-// 700 x 64 36 us, 64 x 64 8.9 us (27).  The same scheme with 16 x 4 lines of a
-// 7-point grid per wavefront took 117 us at 128^3 with the factors in the
-// Infinity Cache but 150 us without, no better than the general sweep's 140 us:
-// 22 strips on the critical path, 198 cycles a step for the second lane shift
-// and its imports, and only 16 steps of coefficients in flight.
+// steps a strip, and 3.9 (64 x 700) to 5.1 us (1000 x 1000) from strip to strip, of
+// which the 64 steps between their first lines are 2.6 us; HBM traffic, 24 *
+// steps / nx + 16 bytes a row in double (40 on long lines, 70 with nx = 64), is far
+// below.  One wavefront per strip and workgroup, because two in one workgroup slowed
+// each other (60 against 78 ns a step).  Per sweep in double, against the
+// general sweep's tiles: 256 x 256 28 to 32 us (88), 301 x 173 28 us (80), 700 x 64
+// 35 us, 64 x 64 9.2 us (27), 64 x 700 47 us, 1000 x 1000 125 us, 8000 x 66 381 us.
+// A sweep that also forms dot(w, y) is bound by its loader: 58 us at 256 x 256.
+// The same scheme with 16 x 4 lines of a 7-point grid per wavefront took 117 us
+// at 128^3 with the factors in the Infinity Cache but 150 us without, no better
+// than the general sweep's 140 us: 22 strips on the critical path, 198 cycles a step
+// for the second lane shift and its imports, and only 16 steps of coefficients in
+// flight.
 #include "buffer_dev.hpp"
 #include "m4g_device.hpp"
 #include "lines.hpp"
@@ -234,10 +238,9 @@ struct LineArgs {
 // longest chain of additions stays as short.
 //
 // The compute wavefront's pace is its number of instructions (about 7 cycles
-// each, alone on its SIMD), so it does nothing else and shares its SIMD with no
-// polling loop.  The hardware spreads the eight wavefronts evenly over the
-// SIMDs, but in no fixed order: each says which SIMD it is on, and the other
-// roles go to wavefronts elsewhere where there are enough.
+// each, alone on its SIMD), so it does nothing else.  The other roles go to wavefronts on
+// other SIMDs, as in the general sweep, though fixed roles measure the same here
+// (64 x 700: 47.6 and 48.0 us, 1000 x 1000: 123.9 and 123.7).
 enum LineRole { kLineCompute, kLineLoad, kLineStore, kLineImport, kLineExport, kLineIdle };
 
 __device__ inline LineRole line_role(const int* simd, int wave)
@@ -502,7 +505,7 @@ __global__ __launch_bounds__(kLineWaves * kWave) void k_line_sweep(LineArgs a, c
         // ---- importer ----
         // The strip before publishes its last line in order.  kPolls polls of the 64 entries after the first missing one
         // are in flight: a consumer that runs at its producer's pace ends up behind by the longest time a value takes,
-        // and that includes the time between two polls.
+        // and that includes the time between two polls (64 x 700: 47.6 us, with one in flight 48.9).
         lds_barrier();
         if (!first) {
             constexpr int kPolls = 3;

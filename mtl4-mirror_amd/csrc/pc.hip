@@ -325,11 +325,15 @@ __device__ inline int sweep_role(const int* simd, int wave)
 // The compute wavefront so issues no global memory operation: its pace is
 // set by LDS and arithmetic latency only.  A sweep is bound by its chain of
 // dependent steps and of hand-overs between tiles, not by bytes.  Eight
-// wavefronts with the roles placed by SIMD and three polls in flight, against
-// five wavefronts in fixed roles with one poll at a time (one IC(0) or ILU(0) sweep
-// in double, median): 7-point grid of 128^3 140.7 -> 128.3 us, 27-point
-// grid of 96^3 315.8 -> 284.4 us (with rows in one piece of 13, see
-// sweep_piece_width), a mesh of 64 400 vertices 174.3 -> 174.9 us.
+// wavefronts with the roles placed by SIMD and three unconditional polls in
+// flight, against five wavefronts in fixed roles with one poll at a time (one IC(0)
+// or ILU(0) sweep in double, median): 7-point grid of 128^3 140.7 -> 128.3 us,
+// 27-point grid of 96^3 315.8 -> 284.4 us (with rows in one piece of 13, see
+// sweep_piece_width), a mesh of 49 384 vertices 174.3 -> 174.9 us.  Of that, the
+// placing gives 0.5 to 1 % (129.5 -> 128.9, 287.9 -> 285.8, 176.5 -> 174.6 us).
+// Three polls instead of one help where few tiles run (BiCGStab on 61 x 53 x 47,
+// 27-point: 13.1 -> 12.9 ms) and cost where all do (96^3: 273.5 -> 285.5 us, 128^3:
+// 128.1 -> 129.0 us).
 template <typename FV, typename VT, bool UNIT, int W>
 __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4* __restrict__ recs,
                                                          const VT* __restrict__ v, VT* __restrict__ y, VT* xbuf,
@@ -459,9 +463,10 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(SweepArgs a, const int4
         // Polls the next imports of the tile, in first-use order, straight
         // from the exchange buffer into LDS and publishes the prefix that has
         // arrived.  Each poll reads the 64 * kImportDepth after progress;
-        // kImportPolls are in flight, because a tile that runs at the pace of
-        // the one before ends up behind by the longest time a value takes,
-        // and that includes the time between two polls.  A poll that finds
+        // kImportPolls are in flight (what they give and cost: above), so that
+        // a tile that runs at the pace of the one before, and ends up behind
+        // by the longest time a value takes, waits less for a next poll.  A
+        // poll that finds
         // nothing new touches no LDS (the window's slots stay in registers,
         // the first missing import comes from ballots), so it does not queue
         // behind the compute wavefront's LDS traffic.
