@@ -2,7 +2,9 @@
  *
  * These functions need no GPU.  They expose the schedule compiler of the
  * triangular sweeps so that its output can be checked on the CPU: they build
- * the tile-pipelined plans exactly as m4g_pc_create does, validate them, and
+ * the tile-pipelined plans exactly as m4g_pc_create does for the factors that it
+ * sweeps in tiles (a 2D grid's whole 5-point pattern is swept line by line
+ * there, without a plan; here it is planned as any other), validate them, and
  * execute them on the host with the kernel's operation order.  No reference
  * counterpart: the reference runs its sweeps sequentially
  * (lower_trisolve.hpp:172-209, upper_trisolve.hpp:159-176).
